@@ -266,3 +266,126 @@ def tolerance(case):
     if f == "lstm":
         return {"rel": 1e-5, "max": 1e-3}      # 7e-7 and 2e-4 (small second moments) after three steps
     return {"rel": 1e-5}
+
+
+# ---------------------------------------------------------------------------------------------------------------------
+# the same results in 64 bits
+# ---------------------------------------------------------------------------------------------------------------------
+def _double(a, dtype="f32", grad=False):
+    t = torch.from_numpy(np.ascontiguousarray(a))
+    if dtype == "bf16":
+        t = t.bfloat16()
+    return t.double().requires_grad_(grad) if t.is_floating_point() else t.long()
+
+
+def _layer_norm64(x, scale, bias, eps):
+    return torch.nn.functional.layer_norm(x, x.shape[-1:], scale, bias, eps)
+
+
+def _gelu64(x):
+    return torch.nn.functional.gelu(x, approximate="tanh")
+
+
+def _exact_mlp(p, steps):
+    w1, b1, w2, b2, x, y = [_double(a) for a in p.inputs]
+    for _ in range(steps):
+        params = [t.detach().requires_grad_(True) for t in (w1, b1, w2, b2)]
+        loss = torch.nn.functional.cross_entropy(torch.relu(x @ params[0] + params[1]) @ params[2] + params[3], y)
+        w1, b1, w2, b2 = [(t - 0.01 * g).detach() for t, g in zip(params, torch.autograd.grad(loss, params))]
+    return [w1, b1, w2, b2, loss.detach()]
+
+
+def _exact_embedding(p):
+    table, idx, upstream = [_double(a) for a in p.inputs]
+    return [table[idx], torch.zeros_like(table).index_add_(0, idx, upstream)]
+
+
+def _exact_resnet18(p, train):
+    A = {n: _double(a, grad=train and n not in ("x", "y") and not n.startswith("mom.")) for n, a in zip(p.input_names, p.inputs)}
+
+    def conv(name, h, stride):
+        w = A[name + ".kernel"].permute(3, 2, 0, 1)
+        total = max((-(-h.shape[2] // stride) - 1) * stride + w.shape[2] - h.shape[2], 0)
+        return torch.nn.functional.conv2d(torch.nn.functional.pad(h, (total // 2, total - total // 2) * 2), w, stride=stride)
+
+    def norm(name, h):
+        return torch.nn.functional.batch_norm(h, None, None, A[name + ".scale"], A[name + ".bias"], training=True, eps=1e-5)
+
+    h = torch.relu(norm("bn_init", conv("conv_init", A["x"].permute(0, 3, 1, 2), 1)))
+    for stage in range(1, 5):
+        for block in (1, 2):
+            q, stride = "stage%d_block%d" % (stage, block), 2 if stage > 1 and block == 1 else 1
+            y = torch.relu(norm(q + ".bn1", conv(q + ".conv1", h, stride)))
+            y = norm(q + ".bn2", conv(q + ".conv2", y, 1))
+            if q + ".conv_proj.kernel" in A:
+                h = norm(q + ".bn_proj", conv(q + ".conv_proj", h, stride))
+            h = torch.relu(h + y)
+    logits = h.mean((2, 3)) @ A["dense.kernel"] + A["dense.bias"]
+    loss = torch.nn.functional.cross_entropy(logits, A["y"])
+    if not train:
+        return [logits, loss]
+    names = [n[4:] for n in p.output_names if n.startswith("mom.")]
+    return list(torch.autograd.grad(loss, [A[n] for n in names])) + [loss.detach()]
+
+
+def _exact_encoder(p, case):
+    A = {n: _double(a, d) for n, a, d in zip(p.input_names, p.inputs, p.input_dtypes)}
+    batch, seq, heads, dim = case["batch"], case["seq"], case["heads"], case["head_dim"]
+    x = _layer_norm64(A["word_emb"][A["input_ids"]] + A["pos_emb"][:seq], A["emb_ln.scale"], A["emb_ln.bias"], 1e-12)
+    masked = (A["attention_mask"] == 0)[:, None, None, :]
+    for n in range(case["layers"]):
+        def linear(t, name):
+            return t @ A["layer%d.%s.kernel" % (n, name)] + A["layer%d.%s.bias" % (n, name)]
+
+        def norm(t, name):
+            return _layer_norm64(t, A["layer%d.%s.scale" % (n, name)], A["layer%d.%s.bias" % (n, name)], 1e-12)
+
+        q, k, v = linear(x, "qkv").reshape(batch, seq, 3, heads, dim).permute(2, 0, 3, 1, 4).contiguous()
+        probs = torch.softmax((q @ k.transpose(2, 3).contiguous() / math.sqrt(dim)).masked_fill(masked, -math.inf), -1)
+        x = norm(x + linear((probs @ v).transpose(1, 2).reshape(batch, seq, heads * dim), "out"), "sa_ln")
+        x = norm(x + linear(_gelu64(linear(x, "ffn1")), "ffn2"), "out_ln")
+    return [x]
+
+
+def _exact_lstm(p, case):
+    params = [_double(a, grad=True) for a in p.inputs[:5]]
+    xs, y = _double(p.inputs[-2]), _double(p.inputs[-1])
+    wi, wh, bias, wo, bo = params
+    h = c = torch.zeros(case["batch"], case["hidden"], dtype=torch.float64)
+    for x in xs:
+        i, f, g, o = (x @ wi + h @ wh + bias).chunk(4, 1)
+        c = torch.sigmoid(f) * c + torch.sigmoid(i) * torch.tanh(g)
+        h = torch.sigmoid(o) * torch.tanh(c)
+    loss = torch.nn.functional.cross_entropy(h @ wo + bo, y)
+    grads = torch.autograd.grad(loss, params)
+    # Adam's first step: its moments start at zero
+    mu, nu = [0.1 * g for g in grads], [0.001 * g * g for g in grads]
+    new = [(t - 1e-3 * (m / 0.1) / (torch.sqrt(v / 0.001) + 1e-8)).detach() for t, m, v in zip(params, mu, nu)]
+    return new + mu + nu + [None, loss.detach()]
+
+
+_EXACT_OPS = {
+    "softmax": lambda x: [torch.softmax(x, -1)],
+    "exp": lambda x: [torch.exp(x)],
+    "add": lambda x, y: [x + y],
+    "sum": lambda x: [x.sum()],
+    "column_stats": lambda x: [x.sum(0), (x * x).sum(0)],
+    "layernorm_bf16": lambda x, scale, bias: [_layer_norm64(x, scale, bias, 1e-12)],
+    "bias_gelu_bf16": lambda x, bias: [_gelu64(x + bias)],
+}
+
+
+def exact(case, seed):
+    p = _program(case, seed)
+    f = case["family"]
+    if f == "mlp":
+        return _exact_mlp(p, case["steps"])
+    if f == "embedding":
+        return _exact_embedding(p)
+    if f == "resnet18":
+        return _exact_resnet18(p, case["train"])
+    if f == "distilbert":
+        return _exact_encoder(p, case)
+    if f == "lstm":
+        return _exact_lstm(p, case)
+    return _EXACT_OPS[case["op"]](*[_double(a, d) for a, d in zip(p.inputs, p.input_dtypes)])
