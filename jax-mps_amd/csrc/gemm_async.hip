@@ -41,9 +41,11 @@ namespace {
 typedef unsigned short u16;
 typedef unsigned int u32;
 typedef float float16v __attribute__((ext_vector_type(16)));
+typedef float float4v __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef short short4v __attribute__((ext_vector_type(4)));
 typedef short short8v __attribute__((ext_vector_type(8)));
+typedef u32 uint4v __attribute__((ext_vector_type(4)));   // (an array of HIP's uint4 structs ended up in scratch memory)
 
 #define GLOBAL_PTR(p) ((__attribute__((address_space(1))) void*)(p))
 #define LDS_PTR(p) ((__attribute__((address_space(3))) void*)(p))
@@ -64,6 +66,19 @@ struct AsyncArgs {
 };
 
 __device__ __forceinline__ u16 to_bf16(float f) { return __builtin_bit_cast(u16, (__bf16)f); }
+
+// a bf16 result as it is stored: bias added to the rounded product, then the activation
+__device__ __forceinline__ u16 finishBf16(const AsyncArgs& g, float v, float bias) {
+  u16 r = to_bf16(v);
+  if (g.bias) r = to_bf16(__uint_as_float((u32)r << 16) + bias);
+  if (g.act == 1) {
+    const float x = __uint_as_float((u32)r << 16);
+    const float u = g.actC * (x + g.actB * (x * x * x));
+    const float ex = __expf(2.f * fminf(u, 20.f));   // 1 + tanh(u) = 2 e^(2u) / (1 + e^(2u)): no cancellation for negative u
+    r = to_bf16(g.actA * x * (2.f * ex * __builtin_amdgcn_rcpf(1.f + ex)));
+  }
+  return r;
+}
 
 // s_waitcnt immediate for "at most n vector-memory operations outstanding" (gfx9 encoding:
 // vmcnt in bits 3:0 and 15:14, expcnt 6:4 and lgkmcnt 11:8 left at their maxima)
@@ -263,18 +278,7 @@ __global__ void __launch_bounds__(WM * 128) gemm_bf16_async(AsyncArgs g) {
   __builtin_amdgcn_s_waitcnt(vmcntImm(0));   // drain the tail loads before the workgroup's LDS is released
 
   const long long cBase = bz * g.M * g.N;
-  // value of accumulator element e of tile (i, j) as it is stored: bias added to the rounded product, then the activation
-  auto finish16 = [&](float v, float bias) -> u16 {
-    u16 r = to_bf16(v);
-    if (g.bias) r = to_bf16(__uint_as_float((u32)r << 16) + bias);
-    if (g.act == 1) {
-      const float x = __uint_as_float((u32)r << 16);
-      const float u = g.actC * (x + g.actB * (x * x * x));
-      const float ex = __expf(2.f * fminf(u, 20.f));   // 1 + tanh(u) = 2 e^(2u) / (1 + e^(2u)): no cancellation for negative u
-      r = to_bf16(g.actA * x * (2.f * ex * __builtin_amdgcn_rcpf(1.f + ex)));
-    }
-    return r;
-  };
+  auto finish16 = [&](float v, float bias) { return finishBf16(g, v, bias); };
   if (g.outBf16 && (g.N & 7) == 0 && ((uintptr_t)g.c & 15) == 0) {
     // bf16 results leave through LDS: an accumulator lane holds 16 rows of one column, so direct stores are
     // 2-byte writes, 64 of them per instruction.  Each 64-row band of the tile is transposed through a ring
@@ -324,6 +328,159 @@ __global__ void __launch_bounds__(WM * 128) gemm_bf16_async(AsyncArgs g) {
           else ((float*)g.c)[cBase + row * g.N + col] = acc[i][j][e] + bias;
         }
       }
+    }
+  }
+}
+
+// Few output tiles: one request of a serving program has 37 rows, and 64x64 tiles of a 768-column product are then twelve
+// workgroups that walk all of K in sequence (bound by the latency of one slab after another).  Here a workgroup owns
+// 16 TMB x 32 of the result and its wavefronts share out the 32-wide slabs of K: each keeps four slabs of both
+// operands in flight in registers, multiplies on its own (no barrier in the loop) and the partial tiles are added in wavefront
+// order through LDS at the end, followed by the usual epilogue.  A k-contiguous operand goes from memory to the MFMA
+// registers directly; an n-contiguous B takes a turn through LDS private to the wavefront ([k][32 columns], rows 96 bytes
+// apart so that a transposing read meets every bank once).  16x16x32 products, because a load instruction then takes 64 bytes
+// from each of 16 rows; with 32x32x16 ones it takes 32 bytes from 32 rows and the L1's line lookups bound the loop, and 37 rows
+// pad to 48 instead of 64.
+// Four wavefronts: eight shorten the chain no further (a unit's loads bound it: 9.0 us against 8.4 for 37 x 3072 x 768) and
+// sixteen lose.  37 rows, K x N: 768x768 5.8 -> 4.4 us, 3072x768 22.5 -> 8.4, 768x2304 8.1 -> 5.0, 768x3072 8.2 -> 5.6.
+constexpr int kFewWaves = 4;
+
+template <int TMB, bool BNN>
+__global__ void __launch_bounds__(kFewWaves * 64) gemm_bf16_few(AsyncArgs g) {
+  constexpr int NW = kFewWaves;
+  constexpr int kDepth = 4, kRow = 96, kSlabBytes = 32 * kRow;
+  constexpr int kTile = 16 * TMB * 32;
+  constexpr int kBytes = BNN && 2 * kSlabBytes > kTile * 4 ? 2 * kSlabBytes : kTile * 4;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[NW * kBytes];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  unsigned id = blockIdx.x;
+  const unsigned total = (unsigned)g.total;
+  if ((total & 7u) == 0) id = (id & 7u) * (total >> 3) + (id >> 3);   // neighbouring column tiles, which share cache lines of B, on one XCD
+  const unsigned perBatch = (unsigned)g.tilesM * (unsigned)g.tilesN;
+  const unsigned bz = id / perBatch, t = id - bz * perBatch;
+  const unsigned tn = t / (unsigned)g.tilesM, tm = t - tn * (unsigned)g.tilesM;
+  const long long b0 = bz / (unsigned)g.batch1, b1 = bz - (unsigned)b0 * (unsigned)g.batch1;
+  const u16* A = g.a + b0 * g.aB0 + b1 * g.aB1;
+  const u16* B = g.b + b0 * g.bB0 + b1 * g.bB1;
+  const long long m0 = (long long)tm * (16 * TMB), n0 = (long long)tn * 32;
+
+  // rows and columns past the edge re-read the last ones; what they produce is not stored
+  const u16* srcA[TMB];
+#pragma unroll
+  for (int i = 0; i < TMB; ++i) {
+    long long m = m0 + i * 16 + (lane & 15);
+    if (m > g.M - 1) m = g.M - 1;
+    srcA[i] = A + m * g.aLd + (lane >> 4) * 8;
+  }
+  const u16* srcB[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    if (BNN) {
+      long long n = n0 + (lane & 3) * 8;
+      if (n > g.N - 8) n = g.N - 8;
+      srcB[j] = B + (long long)(16 * j + (lane >> 2)) * g.bLd + n;
+    } else {
+      long long n = n0 + 16 * j + (lane & 15);
+      if (n > g.N - 1) n = g.N - 1;
+      srcB[j] = B + n * g.bLd + (lane >> 4) * 8;
+    }
+  }
+  const int slabs = (int)(g.K / 32), firstSlab = slabs * wave / NW, mine = slabs * (wave + 1) / NW - firstSlab;
+  uint4v ra[kDepth][TMB], rb[kDepth][2];
+  auto load = [&](auto set, int it) {
+    constexpr int S = decltype(set)::value;
+    int slab = firstSlab + it;
+    if (slab > slabs - 1) slab = slabs - 1;        // past the end: a re-read nobody uses
+    const long long k0 = (long long)slab * 32;
+    const long long kB = BNN ? k0 * g.bLd : k0;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) rb[S][j] = *(const uint4v*)(srcB[j] + kB);
+#pragma unroll
+    for (int i = 0; i < TMB; ++i) ra[S][i] = *(const uint4v*)(srcA[i] + k0);
+  };
+  float4v acc[TMB][2];
+#pragma unroll
+  for (int i = 0; i < TMB; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = (float4v){0};
+  unsigned char* const own = lds + wave * kBytes;
+  const int d = lane & 15;
+  auto multiply = [&](auto set) {
+    constexpr int S = decltype(set)::value;
+    bf16x8 bv[2];
+    if (BNN) {
+      unsigned char* const slab = own + (S & 1) * kSlabBytes;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) *(uint4v*)(slab + (16 * j + (lane >> 2)) * kRow + (lane & 3) * 16) = rb[S][j];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // the wavefront's own LDS accesses stay in this order
+      const unsigned char* const at = slab + (8 * (lane >> 4) + (d >> 2)) * kRow + (d & 3) * 8;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        short4v q[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          q[h] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4v*)(at + 4 * h * kRow + 32 * j));
+        bv[j] = __builtin_bit_cast(bf16x8, (short8v)__builtin_shufflevector(q[0], q[1], 0, 1, 2, 3, 4, 5, 6, 7));
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    } else {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) bv[j] = __builtin_bit_cast(bf16x8, rb[S][j]);
+    }
+#pragma unroll
+    for (int i = 0; i < TMB; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, ra[S][i]), bv[j], acc[i][j], 0, 0, 0);
+  };
+  load(Const<0>(), 0);
+  load(Const<1>(), 1);
+  load(Const<2>(), 2);
+  load(Const<3>(), 3);
+  int it = 0;
+  for (; it + 3 < mine; it += 4) {
+    multiply(Const<0>()); load(Const<0>(), it + 4);
+    multiply(Const<1>()); load(Const<1>(), it + 5);
+    multiply(Const<2>()); load(Const<2>(), it + 6);
+    multiply(Const<3>()); load(Const<3>(), it + 7);
+  }
+  if (it < mine) multiply(Const<0>());
+  if (it + 1 < mine) multiply(Const<1>());
+  if (it + 2 < mine) multiply(Const<2>());
+
+  __syncthreads();                     // the slabs are read: their LDS takes the partial tiles
+  float* const part = (float*)lds;     // [wavefront][row][32]
+#pragma unroll
+  for (int i = 0; i < TMB; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) part[wave * kTile + (i * 16 + (lane >> 4) * 4 + e) * 32 + 16 * j + (lane & 15)] = acc[i][j][e];
+  __syncthreads();
+  const long long cBase = (long long)bz * g.M * g.N;
+#pragma unroll
+  for (int u = tid; u < kTile / 2; u += NW * 64) {
+    const long long row = m0 + (u >> 4), col = n0 + (u & 15) * 2;
+    if (row >= g.M || col >= g.N) continue;
+    float2 v = *(const float2*)(part + 2 * u);
+#pragma unroll
+    for (int w = 1; w < NW; ++w) {
+      const float2 o = *(const float2*)(part + w * kTile + 2 * u);
+      v.x += o.x; v.y += o.y;
+    }
+    const bool two = col + 1 < g.N;
+    const long long at = cBase + row * g.N + col;
+    if (g.outBf16) {
+      float x = 0.f, y = 0.f;
+      if (g.bias) {
+        x = __uint_as_float((u32)((const u16*)g.bias)[col] << 16);
+        if (two) y = __uint_as_float((u32)((const u16*)g.bias)[col + 1] << 16);
+      }
+      ((u16*)g.c)[at] = finishBf16(g, v.x, x);
+      if (two) ((u16*)g.c)[at + 1] = finishBf16(g, v.y, y);
+    } else {
+      const float* bias = (const float*)g.bias;
+      ((float*)g.c)[at] = v.x + (bias ? bias[col] : 0.f);
+      if (two) ((float*)g.c)[at + 1] = v.y + (bias ? bias[col + 1] : 0.f);
     }
   }
 }
@@ -438,9 +595,55 @@ extern "C" size_t mi355_gemm_bf16_async_workspace_bytes(const mi355_gemm_desc* d
   return bytes;
 }
 
+// The kernel for few output tiles of 16-bit products whose lhs rows are k-contiguous and whose rhs is contiguous either way, all
+// 16-byte loads, K in whole slabs (0 = launched, -1 = not one of its shapes).
+static int launchFew(const mi355_gemm_desc* d, const void* a, const void* b, void* c, const void* bias, hipStream_t st) {
+  if (d->in_dtype != 1 || (d->out_dtype != 0 && d->out_dtype != 1) || (d->act && d->out_dtype != 1)) return -1;
+  const long long nb = d->batch0 * d->batch1;
+  if (d->M <= 0 || d->N <= 0 || d->K <= 0 || nb <= 0 || nb > 65535 || d->K % 32 != 0) return -1;
+  if (d->aCol != 1 || d->aRow % 8 || !aligned16(a) || !aligned16(b)) return -1;
+  const bool rowsOfK = d->bCol == 1 && d->bRow % 8 == 0 && d->N % 8 == 0 && d->bRow >= d->N;
+  const bool kContiguous = d->bRow == 1 && d->bCol % 8 == 0;
+  if (!rowsOfK && !kContiguous) return -1;
+  if (d->batch0 > 1 && (d->aB0 % 8 || d->bB0 % 8)) return -1;
+  if (d->batch1 > 1 && (d->aB1 % 8 || d->bB1 % 8)) return -1;
+  // While every workgroup of 64 rows has a compute unit of its own.  Measured against the 64x64 tiles of the ring kernel
+  // (K x N: us at the largest M inside the line, then at the next one): 768x768 7.5 / 8.4 at M = 512, 10.9 / 8.4 at 768;
+  // 3072x768 18.1 / 23.5 at 512, 33 / 23.5 at 768; 768x2304 7.6 / 8.3 at 192, 11.2 / 8.7 at 256; 768x3072 7.8 / 8.3 at 128,
+  // 10.9 / 8.6 at 192.
+  constexpr long long kUnits = 256;
+  const long long blocks = (d->M + 15) / 16, tilesN = (d->N + 31) / 32;
+  if ((blocks + 3) / 4 * tilesN * nb > kUnits) return -1;
+  AsyncArgs g;
+  g.a = (const u16*)a; g.b = (const u16*)b; g.c = c; g.bias = bias;
+  g.M = d->M; g.N = d->N; g.K = d->K;
+  g.aB0 = d->aB0; g.aB1 = d->aB1; g.aLd = d->aRow;
+  g.bB0 = d->bB0; g.bB1 = d->bB1; g.bLd = rowsOfK ? d->bRow : d->bCol;
+  g.batch1 = (int)d->batch1;
+  g.outBf16 = d->out_dtype == 1;
+  g.act = d->act; g.actA = d->act_a; g.actB = d->act_b; g.actC = d->act_c;
+  // the fewest rows per workgroup that still give each a unit of its own: a unit takes in about 15 bytes a cycle here, so what
+  // one of them has to read sets the time (37 rows, 3072x768: 13.7 us as one tile row of 48, 8.4 as three of 16)
+  int tmb = 1;
+  while ((blocks + tmb - 1) / tmb * tilesN * nb > kUnits) ++tmb;
+  g.tilesM = (int)((blocks + tmb - 1) / tmb);
+  g.tilesN = (int)tilesN;
+  g.total = (long long)g.tilesM * g.tilesN * nb;
+  const dim3 grid((unsigned)g.total);
+#define FEW(TMB) do { \
+  if (rowsOfK) gemm_bf16_few<TMB, true><<<grid, kFewWaves * 64, 0, st>>>(g); else gemm_bf16_few<TMB, false><<<grid, kFewWaves * 64, 0, st>>>(g); } while (0)
+  if (tmb == 1) FEW(1); else if (tmb == 2) FEW(2); else if (tmb == 3) FEW(3); else FEW(4);
+#undef FEW
+  return hipGetLastError() == hipSuccess ? 0 : 3;
+}
+
 // 0 = launched, -1 = layout does not qualify, other = launch error.
 extern "C" int mi355_gemm_bf16_async(const mi355_gemm_desc* d, const void* a, const void* b, void* c, const void* bias, void* workspace,
                                      size_t workspace_bytes, mi355_stream_t s) {
+  static const char* force = getenv("MI355X_GEMM_TILE");   // "256x128", "128x128", "128x64", "64x64": tuning aid
+  const int wideMode = getenv("MI355X_GEMM_WIDE") ? atoi(getenv("MI355X_GEMM_WIDE")) : 1;   // read at every call: tests switch it
+  if (!force && wideMode == 1)                             // (a forced tiling is one of the ring kernel's)
+    if (const int few = launchFew(d, a, b, c, bias, (hipStream_t)s); few >= 0) return few;
   OperandPlan pa, pb;
   if (!qualifies(d, pa, pb)) return -1;
   if (!aligned16(a) || !aligned16(b)) return -1;
@@ -472,7 +675,6 @@ extern "C" int mi355_gemm_bf16_async(const mi355_gemm_desc* d, const void* a, co
   auto tiles = [&](int bm, int bn) { return ((d->M + bm - 1) / bm) * ((d->N + bn - 1) / bn) * nb; };
   // the largest tile that still leaves about three workgroups per compute unit
   int bm = 64, bn = 64;
-  static const char* force = getenv("MI355X_GEMM_TILE");   // "256x128", "128x128", "128x64", "64x64": tuning aid
   if (force) sscanf(force, "%dx%d", &bm, &bn);
   else if (d->M > 128 && d->N > 64 && tiles(256, 128) >= 1024) { bm = 256; bn = 128; }
   // an in-place n-contiguous rhs wants twice as many 128x128 tiles before they pay (measured: 4096x768x3072 runs
@@ -485,7 +687,6 @@ extern "C" int mi355_gemm_bf16_async(const mi355_gemm_desc* d, const void* a, co
   // (N = 768) much slower.  One 64 KB stage in flight per compute unit does not cover the load latency (about 5 500
   // cycles per 64 of K against 2 048 of products), and the 160 KB of LDS hold no third stage of this tile.
   // MI355X_GEMM_WIDE=0 never, =2 whenever the shape allows.
-  const int wideMode = getenv("MI355X_GEMM_WIDE") ? atoi(getenv("MI355X_GEMM_WIDE")) : 1;   // read at every call: tests switch it
   bool wide = false;
   if (!force && wideMode != 0 && d->M >= 256 && d->N >= 256)
     wide = wideMode == 2 || (tiles(256, 256) >= 192 && d->K >= 2048);
