@@ -414,7 +414,10 @@ typedef unsigned int uint4v __attribute__((ext_vector_type(4)));
 constexpr unsigned kOutside = 0x80000000u;     // an offset no tensor reaches (tensors stay below 2 GiB here)
 constexpr int kTapTableBytes = 16384;          // largest per-workgroup tap table
 
-template <int BM, int BN, int AMODE, int BMODE, bool TABLE>
+// RAGGED: the features do not fill whole k-tiles (C is no multiple of 16: the batch of a filter gradient, narrow layers).  The
+// last tile of a tap is then fetched with the offset that reads as zero in the lanes past C: one compare and select per fetch,
+// which the other problems do not pay.
+template <int BM, int BN, int AMODE, int BMODE, bool TABLE, bool RAGGED>
 __device__ __forceinline__ void leanBody(const ConvP& p, int split) {
   constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 32, TN = WN / 32;
   constexpr int NA4 = BM / 64, NB4 = BN / 64;
@@ -521,10 +524,19 @@ __device__ __forceinline__ void leanBody(const ConvP& p, int split) {
     constexpr int S = decltype(setTag)::value;
     const unsigned sA = (unsigned)(AMODE == 1 ? nc : nc * p.lhsF) * 4u;
     const unsigned sB = (unsigned)(BMODE == 1 ? toffB + nc * p.rhsI : toffB + nc) * 4u;
+    const int left = p.C - nc;                // features of this tap from the tile's first on
 #pragma unroll
-    for (int i = 0; i < NA4; ++i) ra[S][i] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rsA, (int)aV[i], (int)sA, 0));
+    for (int i = 0; i < NA4; ++i) {
+      const int k = AMODE == 1 ? aKq : tid / (BM / 4) + (1024 / BM) * i;
+      const unsigned v = RAGGED && k >= left ? kOutside : aV[i];
+      ra[S][i] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rsA, (int)v, (int)sA, 0));
+    }
 #pragma unroll
-    for (int i = 0; i < NB4; ++i) rb[S][i] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rsB, (int)bV[i], (int)sB, 0));
+    for (int i = 0; i < NB4; ++i) {
+      const int k = BMODE == 2 ? aKq : tid / (BN / 4) + (1024 / BN) * i;
+      const unsigned v = RAGGED && k >= left ? kOutside : bV[i];
+      rb[S][i] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rsB, (int)v, (int)sB, 0));
+    }
     nc += BK;
     if (nc >= p.C) {
       nc = 0;
@@ -690,9 +702,9 @@ __device__ __forceinline__ void leanBody(const ConvP& p, int split) {
   }
 }
 
-template <int BM, int BN, int AMODE, int BMODE, bool TABLE>
+template <int BM, int BN, int AMODE, int BMODE, bool TABLE, bool RAGGED>
 __global__ void __launch_bounds__(256, wavesPerSimd(BM, BN, AMODE, BMODE)) conv_igemm_lean(ConvP p) {
-  leanBody<BM, BN, AMODE, BMODE, TABLE>(p, (int)blockIdx.z);
+  leanBody<BM, BN, AMODE, BMODE, TABLE, RAGGED>(p, (int)blockIdx.z);
 }
 
 // Several unsplit problems of one convolution (the residue classes of an input-dilated one) as one launch:
@@ -702,7 +714,7 @@ struct ConvPack { ConvP c[kMaxPack]; };
 
 template <int BM, int BN, int AMODE, int BMODE, bool TABLE>
 __global__ void __launch_bounds__(256, wavesPerSimd(BM, BN, AMODE, BMODE)) conv_igemm_lean_pack(ConvPack ps) {
-  leanBody<BM, BN, AMODE, BMODE, TABLE>(ps.c[blockIdx.z], 0);
+  leanBody<BM, BN, AMODE, BMODE, TABLE, false>(ps.c[blockIdx.z], 0);   // (residue classes need whole k-tiles: partsOf)
 }
 
 // out(m, n) = sum over splits of partial[s][m][n].  32 consecutive outputs per workgroup, the
@@ -776,7 +788,7 @@ __global__ void __launch_bounds__(256) conv_repack_filter(const float* __restric
 struct ConvChoice {
   bool fast = false;
   int amode = 0, bmode = 0, bm = 128, bn = 128, splitK = 1, tilesPerSplit = 0, kTiles = 0, cTiles = 0, bFast = 0;
-  bool kflat = false;
+  bool kflat = false, ragged = false;
 };
 
 bool fitsInt(const mi355_conv_desc* d) {
@@ -792,19 +804,25 @@ ConvChoice choose(const mi355_conv_desc* d, long long tapsVisited = -1, int shar
   long long M = d->N, K = d->C;
   for (int k = 0; k < d->nsp; ++k) { M *= d->out[k]; K *= d->k[k]; }
   long long N = d->O;
-  bool chunk = d->C % BK == 0;
+  // Features in k-tiles of 16 per tap.  A ragged last tile multiplies zeros, at worst (C = 8, 17) as many as features; the
+  // scalar loaders that take any C compute an address and a condition per element and run at a third of the rate
+  // (filter gradients of a batch of 24: 45 us against 18, with a quarter of the products zeros).
+  const bool whole = d->C % BK == 0, ragged = d->C >= 8;
+  const bool kVectors = whole || (ragged && d->C % 4 == 0), rowVectors = whole || ragged;
   auto mult4 = [](long long x) { return x % 4 == 0; };
   long long s0 = d->nsp > 0 ? d->lhsS[0] : 0, s1 = d->nsp > 1 ? d->lhsS[1] : 0;
   long long r0 = d->nsp > 0 ? d->rhsS[0] : 0, r1 = d->nsp > 1 ? d->rhsS[1] : 0;
-  if (chunk && d->lhsF == 1 && mult4(d->lhsB) && mult4(s0) && mult4(s1)) c.amode = 1;
-  else if (chunk && d->lhsB == 1 && d->N % 4 == 0 && mult4(d->lhsF) && mult4(s0) && mult4(s1)) { c.amode = 2; c.bFast = 1; }
-  if (chunk && d->rhsO == 1 && N % 4 == 0 && mult4(d->rhsI) && mult4(r0) && mult4(r1)) c.bmode = 1;
-  else if (chunk && d->rhsI == 1 && mult4(d->rhsO) && mult4(r0) && mult4(r1)) c.bmode = 2;
-  c.kflat = !chunk;
+  if (kVectors && d->lhsF == 1 && mult4(d->lhsB) && mult4(s0) && mult4(s1)) c.amode = 1;
+  else if (rowVectors && d->lhsB == 1 && d->N % 4 == 0 && mult4(d->lhsF) && mult4(s0) && mult4(s1)) { c.amode = 2; c.bFast = 1; }
+  if (rowVectors && d->rhsO == 1 && N % 4 == 0 && mult4(d->rhsI) && mult4(r0) && mult4(r1)) c.bmode = 1;
+  else if (kVectors && d->rhsI == 1 && mult4(d->rhsO) && mult4(r0) && mult4(r1)) c.bmode = 2;
+  if (!whole && (c.amode == 0 || c.bmode == 0)) { c.amode = c.bmode = c.bFast = 0; c.kflat = true; }
+  const bool chunk = !c.kflat;
+  c.ragged = chunk && !whole;
   long long taps = 1;
   for (int k = 0; k < d->nsp; ++k) taps *= d->k[k];
   if (tapsVisited >= 0 && chunk) taps = tapsVisited;
-  c.cTiles = chunk ? (int)(d->C / BK) : 1;
+  c.cTiles = chunk ? (int)((d->C + BK - 1) / BK) : 1;
   c.kTiles = chunk ? (int)(taps * c.cTiles) : (int)((K + BK - 1) / BK);
   // largest tile that still leaves minTiles output tiles (split-K then multiplies the workgroups); tuned on the ResNet18 step
   auto tilesOf = [&](int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
@@ -842,7 +860,8 @@ ConvChoice choose(const mi355_conv_desc* d, long long tapsVisited = -1, int shar
 template <int BM, int BN>
 void launchIgemm(const ConvChoice& c, const ConvP& p, dim3 grid, hipStream_t st) {
 #define CASE(A, B, F) conv_igemm_f32<BM, BN, A, B, F><<<grid, 256, 0, st>>>(p)
-#define LEAN(A, B) do { if (table) conv_igemm_lean<BM, BN, A, B, true><<<grid, 256, table, st>>>(p); else conv_igemm_lean<BM, BN, A, B, false><<<grid, 256, 0, st>>>(p); } while (0)
+#define LEAN_R(A, B, R) do { if (table) conv_igemm_lean<BM, BN, A, B, true, R><<<grid, 256, table, st>>>(p); else conv_igemm_lean<BM, BN, A, B, false, R><<<grid, 256, 0, st>>>(p); } while (0)
+#define LEAN(A, B) do { if (c.ragged) LEAN_R(A, B, true); else LEAN_R(A, B, false); } while (0)
   if (c.kflat) { CASE(0, 0, true); return; }
   const size_t tableBytes = (size_t)p.taps * BM * sizeof(unsigned);
   const unsigned table = tableBytes <= (size_t)kTapTableBytes ? (unsigned)tableBytes : 0u;
@@ -858,6 +877,7 @@ void launchIgemm(const ConvChoice& c, const ConvP& p, dim3 grid, hipStream_t st)
     case 8: LEAN(2, 2); break;
   }
 #undef LEAN
+#undef LEAN_R
 #undef CASE
 }
 
