@@ -1539,7 +1539,11 @@ FusedCode generateReduceKernel(const std::vector<Op*>& reduces, const LeafPredic
   int TY = 256 / TX;
   int64_t gridX = (kvecs + TX - 1) / TX;
   int64_t P = 1;
-  static const int colPerThread = getenv("MI355X_REDUCE_COL_PER_THREAD") ? atoi(getenv("MI355X_REDUCE_COL_PER_THREAD")) : 16;
+  // Sixteen visits per lane are best while that gives workgroups for half the compute units (64 of them: ResNet18's statistics at
+  // batch 16, one wavefront per SIMD walking sixteen dependent-latency loads; its forward pass 559 us with sixteen visits,
+  // 551 with eight, and at batch 128, 512 workgroups, the train step 4716 us with sixteen and 4763 with eight).
+  static const int colEnv = getenv("MI355X_REDUCE_COL_PER_THREAD") ? atoi(getenv("MI355X_REDUCE_COL_PER_THREAD")) : 0;
+  const int colPerThread = colEnv ? colEnv : ((Rn + TY * 16 - 1) / (TY * 16) * gridX < 128 ? 8 : 16);
   if (Rn > (int64_t)TY * 16) P = std::min<int64_t>((Rn + TY * colPerThread - 1) / (TY * colPerThread), std::max<int64_t>(1, 2048 / gridX));
   // a small input is cheaper to walk in one launch (a few dozen loads per lane) than to split over a second, dependent one
   if (Rn * Kn <= reduceOnePassLimit() && Rn <= (int64_t)TY * 128) P = 1;
