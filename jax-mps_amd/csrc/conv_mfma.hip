@@ -69,6 +69,7 @@ struct ConvP {
   // a later pass folds the tile rows in order.  Null when not wanted.
   float* statSum;
   float* statSq;
+  const float* bias;             // N values added to every row of the result (by the fold when K is split), or null
 };
 
 struct Row {
@@ -112,6 +113,7 @@ template <int TM, int TN, int WM, int WN>
 __device__ __forceinline__ void storeAccumulators(const ConvP& p, float16v (&acc)[TM][TN], int m0, int n0, int wm, int wn, int lane, int split) {
   const bool partial = p.splitK > 1;
   const bool vec = p.outVec != 0;
+  const float* const bias = partial ? nullptr : p.bias;
 #pragma unroll
   for (int a = 0; a < TM; ++a) {
     const int m = m0 + wm * WM + a * 32 + (lane & 31);
@@ -134,12 +136,18 @@ __device__ __forceinline__ void storeAccumulators(const ConvP& p, float16v (&acc
       for (int g4 = 0; g4 < 4; ++g4) {
         const int n = n0 + wn * WN + b * 32 + g4 * 8 + (lane >> 5) * 4;
         if (n >= p.N) continue;
+        float v[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          v[r] = acc[a][b][4 * g4 + r];
+          if (bias && n + r < p.N) v[r] += bias[n + r];
+        }
         if (vec) {
-          *(float4*)(p.out + rowOff + n) = make_float4(acc[a][b][4 * g4], acc[a][b][4 * g4 + 1], acc[a][b][4 * g4 + 2], acc[a][b][4 * g4 + 3]);
+          *(float4*)(p.out + rowOff + n) = make_float4(v[0], v[1], v[2], v[3]);
         } else {
 #pragma unroll
           for (int r = 0; r < 4; ++r)
-            if (n + r < p.N) p.out[rowOff + (n + r) * colStride] = acc[a][b][4 * g4 + r];
+            if (n + r < p.N) p.out[rowOff + (n + r) * colStride] = v[r];
         }
       }
     }
@@ -739,6 +747,7 @@ __global__ void __launch_bounds__(256) conv_fold_partials(const float* __restric
   int b, o0, o1;
   if (p.bFast) { b = m % p.Nb; int t = m / p.Nb; o1 = t % p.o1n; o0 = t / p.o1n; }
   else { o1 = m % p.o1n; int t = m / p.o1n; o0 = t % p.o0n; b = t / p.o0n; }
+  if (p.bias) s += p.bias[n];
   out[(long long)b * p.outB + (long long)o0 * p.outS0 + (long long)o1 * p.outS1 + (long long)n * p.outF] = s;
 }
 
@@ -753,6 +762,7 @@ __global__ void __launch_bounds__(256) conv_fold_few(const float* __restrict__ p
     s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
   }
   const int m = (int)(i / p.N), n = (int)(i - (long long)m * p.N);
+  if (p.bias) { s.x += p.bias[n]; s.y += p.bias[n + 1]; s.z += p.bias[n + 2]; s.w += p.bias[n + 3]; }
   int b, o0, o1;
   if (p.bFast) { b = m % p.Nb; int t = m / p.Nb; o1 = t % p.o1n; o0 = t / p.o1n; }
   else { o1 = m % p.o1n; int t = m / p.o1n; o0 = t % p.o0n; b = t / p.o0n; }
@@ -989,7 +999,8 @@ int mi355_conv_direct(const mi355_conv_desc* d, const void* lhs, const void* rhs
 
 // Launches one part; with `prepared` set it only fills the kernel parameters of an unsplit part (returns -1 when the part cannot be prepared that way).
 static int launchPart(const ConvPart& part, const void* lhs, const void* rhs, void* out, void* workspace, size_t workspace_bytes, hipStream_t st,
-                      int sharedLaunch = 1, ConvChoice* preparedChoice = nullptr, ConvP* prepared = nullptr, float* statSum = nullptr, float* statSq = nullptr) {
+                      int sharedLaunch = 1, ConvChoice* preparedChoice = nullptr, ConvP* prepared = nullptr, float* statSum = nullptr, float* statSq = nullptr,
+                      const float* bias = nullptr) {
   const mi355_conv_desc* d = &part.d;
   ConvChoice c = choose(d, part.taps(), sharedLaunch);
   ConvP p;
@@ -997,6 +1008,7 @@ static int launchPart(const ConvPart& part, const void* lhs, const void* rhs, vo
   p.rhs = (const float*)rhs;
   p.statSum = statSum;
   p.statSq = statSq;
+  p.bias = bias;
   p.tilesM = 0;
   p.tilesXY = 0;
   long long M = d->N, K = d->C;
@@ -1099,16 +1111,8 @@ int mi355_conv_stats_rows(const mi355_conv_desc* d) {
   return (int)((M + c.bm - 1) / c.bm);
 }
 
-int mi355_conv_stats(const mi355_conv_desc* d, const void* lhs, const void* rhs, void* out, void* workspace, size_t workspace_bytes,
-                     float* stat_sum, float* stat_sq, mi355_stream_t s);
-
-int mi355_conv(const mi355_conv_desc* d, const void* lhs, const void* rhs, void* out, void* workspace, size_t workspace_bytes,
-               mi355_stream_t s) {
-  return mi355_conv_stats(d, lhs, rhs, out, workspace, workspace_bytes, nullptr, nullptr, s);
-}
-
-int mi355_conv_stats(const mi355_conv_desc* d, const void* lhs, const void* rhs, void* out, void* workspace, size_t workspace_bytes,
-                     float* stat_sum, float* stat_sq, mi355_stream_t s) {
+static int convolve(const mi355_conv_desc* d, const void* lhs, const void* rhs, void* out, void* workspace, size_t workspace_bytes,
+                    float* stat_sum, float* stat_sq, const float* bias, mi355_stream_t s) {
   hipStream_t st = (hipStream_t)s;
   if (stat_sum && mi355_conv_stats_rows(d) == 0) return 5;   // the planner asked for statistics this convolution cannot deliver
   mi355_conv_desc d2;
@@ -1129,7 +1133,7 @@ int mi355_conv_stats(const mi355_conv_desc* d, const void* lhs, const void* rhs,
     workspace_bytes -= repack;
     d = &d2;
   }
-  if (!choose(d).fast) return mi355_conv_direct(d, lhs, rhs, out, s);
+  if (!choose(d).fast) return bias ? -1 : mi355_conv_direct(d, lhs, rhs, out, s);
   const std::vector<ConvPart> parts = partsOf(d);
   static const bool packOff = getenv("MI355X_CONV_PACK") && getenv("MI355X_CONV_PACK")[0] == '0';
   if (parts.size() > 1 && parts.size() <= (size_t)kMaxPack && !packOff) {
@@ -1138,7 +1142,7 @@ int mi355_conv_stats(const mi355_conv_desc* d, const void* lhs, const void* rhs,
     ConvChoice cs[kMaxPack];
     bool ok = true;
     for (size_t i = 0; i < parts.size() && ok; ++i) {
-      ok = launchPart(parts[i], lhs, rhs, out, workspace, workspace_bytes, st, (int)parts.size(), &cs[i], &ps.c[i]) == 0;
+      ok = launchPart(parts[i], lhs, rhs, out, workspace, workspace_bytes, st, (int)parts.size(), &cs[i], &ps.c[i], nullptr, nullptr, bias) == 0;
       if (ok && i > 0) ok = cs[i].amode == cs[0].amode && cs[i].bmode == cs[0].bmode && cs[i].bm == cs[0].bm && cs[i].bn == cs[0].bn && ps.c[i].N == ps.c[0].N;
     }
     if (ok) {
@@ -1151,9 +1155,24 @@ int mi355_conv_stats(const mi355_conv_desc* d, const void* lhs, const void* rhs,
   }
   for (const ConvPart& part : parts) {
     // parts run back to back on the stream, so they can share the split-K scratch
-    if (int r = launchPart(part, lhs, rhs, out, workspace, workspace_bytes, st, 1, nullptr, nullptr, stat_sum, stat_sq)) return r;
+    if (int r = launchPart(part, lhs, rhs, out, workspace, workspace_bytes, st, 1, nullptr, nullptr, stat_sum, stat_sq, bias)) return r;
   }
   return 0;
+}
+
+int mi355_conv(const mi355_conv_desc* d, const void* lhs, const void* rhs, void* out, void* workspace, size_t workspace_bytes,
+               mi355_stream_t s) {
+  return convolve(d, lhs, rhs, out, workspace, workspace_bytes, nullptr, nullptr, nullptr, s);
+}
+
+int mi355_conv_stats(const mi355_conv_desc* d, const void* lhs, const void* rhs, void* out, void* workspace, size_t workspace_bytes,
+                     float* stat_sum, float* stat_sq, mi355_stream_t s) {
+  return convolve(d, lhs, rhs, out, workspace, workspace_bytes, stat_sum, stat_sq, nullptr, s);
+}
+
+int mi355_conv_bias(const mi355_conv_desc* d, const void* lhs, const void* rhs, void* out, const void* bias, void* workspace,
+                    size_t workspace_bytes, mi355_stream_t s) {
+  return convolve(d, lhs, rhs, out, workspace, workspace_bytes, nullptr, nullptr, (const float*)bias, s);
 }
 
 }  // extern "C"

@@ -121,6 +121,10 @@ typedef struct {
 int mi355_conv(const mi355_conv_desc* d, const void* lhs, const void* rhs, void* out, void* workspace,
                size_t workspace_bytes, mi355_stream_t s);
 size_t mi355_conv_workspace_bytes(const mi355_conv_desc* d);
+// The convolution with a value per output feature added to the result (the same sum a later pass over it would make);
+// -1, with nothing launched, where only the direct kernel takes the convolution.  bias may be NULL.
+int mi355_conv_bias(const mi355_conv_desc* d, const void* lhs, const void* rhs, void* out, const void* bias, void* workspace,
+                    size_t workspace_bytes, mi355_stream_t s);
 // Column statistics next to the output: mi355_conv_stats_rows(d) > 0 says the convolution can deliver, for each of that
 // many tile rows i and every output feature n, the sum and the sum of squares of its rows' outputs (stat_sum[i * O + n],
 // stat_sq[i * O + n], both rows x O floats); folding the tile rows in order gives the statistics of the whole output.
