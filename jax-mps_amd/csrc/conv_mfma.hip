@@ -995,6 +995,8 @@ size_t mi355_conv_workspace_bytes(const mi355_conv_desc* d) {
   return repack + most;
 }
 
+int mi355_conv_implicit(const mi355_conv_desc* d) { return choose(d).fast ? 1 : 0; }
+
 int mi355_conv_direct(const mi355_conv_desc* d, const void* lhs, const void* rhs, void* out, mi355_stream_t s);
 
 // Launches one part; with `prepared` set it only fills the kernel parameters of an unsplit part (returns -1 when the part cannot be prepared that way).

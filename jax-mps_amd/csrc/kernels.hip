@@ -1065,7 +1065,8 @@ int mi355_copy_multi_if(int n, void* const* dst, const void* const* src, const s
 
 // An unbatched fp32 GEMM is a convolution without spatial dims (rows = batch, k = input
 // features, columns = output features): it then runs on the implicit-GEMM kernel with its
-// vector tile loaders, register prefetch and split-K for shapes with few output tiles.
+// vector tile loaders, register prefetch and split-K for shapes with few output tiles.  Operands
+// past that kernel's 32-bit offsets stay on the strided tile kernel, which counts in 64 bits.
 static bool gemmAsPointwiseConv(const mi355_gemm_desc* d, mi355_conv_desc* c) {
   if (d->in_dtype != 0 || d->out_dtype != 0 || d->batch0 * d->batch1 != 1 || d->K <= 0) return false;
   *c = mi355_conv_desc{};
@@ -1076,7 +1077,7 @@ static bool gemmAsPointwiseConv(const mi355_gemm_desc* d, mi355_conv_desc* c) {
   c->rhsI = d->bRow; c->rhsO = d->bCol;
   c->outB = d->N; c->outF = 1;
   c->dtype = 0;
-  return true;
+  return mi355_conv_implicit(c) != 0;
 }
 
 // Tile edge of the small-product kernel for this GEMM, 0 when the product is big enough to want
@@ -1225,10 +1226,7 @@ int mi355_gemm(const mi355_gemm_desc* d, const void* a, const void* b, void* c, 
   if (gemmAsPointwiseConv(d, &cd) && (((uintptr_t)a | (uintptr_t)b) & 15) == 0) {
     // the bias rides in the stores (or in the fold of a split K): the pass that added it took 4.5 to 7 us per layer
     // of 1024 rows, a tenth of the products' time
-    int r = d->act ? -1 : mi355_conv_bias(&cd, a, b, c, bias, workspace, workspace_bytes, s);
-    if (r >= 0) return r;
-    r = mi355_conv(&cd, a, b, c, workspace, workspace_bytes, s);
-    return r ? r : addBias(d, c, bias, s);
+    return mi355_conv_bias(&cd, a, b, c, bias, workspace, workspace_bytes, s);
   }
   if (nb > 65535) return 1;   // grid.z limit; callers fold larger batches
   dim3 grid((unsigned)((d->N + 63) / 64), (unsigned)((d->M + 63) / 64), (unsigned)nb);
