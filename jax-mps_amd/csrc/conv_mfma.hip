@@ -801,10 +801,29 @@ struct ConvChoice {
   bool kflat = false, ragged = false;
 };
 
+// Elements from an operand's first to its last one, that included.  Dense operands are as long as they have elements; rows or columns
+// of a slice that is read in place lie further apart than they are long.
+long long lhsExtent(const mi355_conv_desc* d) {
+  if (d->N <= 0 || d->C <= 0) return 0;
+  long long last = (d->N * d->batchGroups - 1) * d->lhsB + (d->C - 1) * d->lhsF;
+  for (int k = 0; k < d->nsp; ++k) { if (d->in[k] <= 0) return 0; last += (d->in[k] - 1) * d->lhsS[k]; }
+  return last + 1;
+}
+
+long long rhsExtent(const mi355_conv_desc* d) {
+  if (d->O <= 0 || d->C <= 0) return 0;
+  long long last = (d->O - 1) * d->rhsO + (d->C - 1) * d->rhsI;
+  for (int k = 0; k < d->nsp; ++k) { if (d->k[k] <= 0) return 0; last += (d->k[k] - 1) * d->rhsS[k]; }
+  return last + 1;
+}
+
+constexpr long long kVectorExtent = 1ll << 29;   // 2 GiB: what the buffer descriptors and byte offsets of the vector-loader kernel reach
+
 bool fitsInt(const mi355_conv_desc* d) {
   long long lhs = d->N * d->batchGroups * d->C, rhs = d->C * d->O, out = d->N * d->O;
   for (int k = 0; k < d->nsp; ++k) { lhs *= d->in[k]; rhs *= d->k[k]; out *= d->out[k]; }
-  return lhs < (1ll << 29) && rhs < (1ll << 29) && out < (1ll << 31);   // inputs below 2 GiB: buffer descriptors and byte offsets are 32-bit
+  // (the scalar loaders' element offsets are 32-bit)
+  return lhs < kVectorExtent && rhs < kVectorExtent && out < (1ll << 31) && lhsExtent(d) < (1ll << 31) && rhsExtent(d) < (1ll << 31);
 }
 
 ConvChoice choose(const mi355_conv_desc* d, long long tapsVisited = -1, int sharedLaunch = 1) {
@@ -817,7 +836,9 @@ ConvChoice choose(const mi355_conv_desc* d, long long tapsVisited = -1, int shar
   // Features in k-tiles of 16 per tap.  A ragged last tile multiplies zeros, at worst (C = 8, 17) as many as features; the
   // scalar loaders that take any C compute an address and a condition per element and run at a third of the rate
   // (filter gradients of a batch of 24: 45 us against 18, with a quarter of the products zeros).
-  const bool whole = d->C % BK == 0, ragged = d->C >= 8;
+  // Slices that reach further than a descriptor stay on the scalar loaders too.
+  const bool reached = lhsExtent(d) < kVectorExtent && rhsExtent(d) < kVectorExtent;
+  const bool whole = reached && d->C % BK == 0, ragged = reached && d->C >= 8;
   const bool kVectors = whole || (ragged && d->C % 4 == 0), rowVectors = whole || ragged;
   auto mult4 = [](long long x) { return x % 4 == 0; };
   long long s0 = d->nsp > 0 ? d->lhsS[0] : 0, s1 = d->nsp > 1 ? d->lhsS[1] : 0;
@@ -1050,11 +1071,7 @@ static int launchPart(const ConvPart& part, const void* lhs, const void* rhs, vo
   }
   p.cTiles = c.cTiles; p.kTiles = c.kTiles; p.splitK = c.splitK; p.tilesPerSplit = c.tilesPerSplit;
   p.taps = part.kc[0] * part.kc[1];
-  {
-    long long lhsN = d->N * d->batchGroups * d->C, rhsN = d->C * d->O;
-    for (int k = 0; k < d->nsp; ++k) { lhsN *= d->in[k]; rhsN *= d->k[k]; }
-    p.lhsBytes = (unsigned)(lhsN * 4); p.rhsBytes = (unsigned)(rhsN * 4);   // below 2 GiB each (fitsInt)
-  }
+  p.lhsBytes = (unsigned)(lhsExtent(d) * 4); p.rhsBytes = (unsigned)(rhsExtent(d) * 4);   // below 2 GiB each where the descriptors are used (choose)
   float* dst = (float*)out + part.outOffset;
   if (c.splitK > 1) {
     size_t need = (size_t)c.splitK * (size_t)M * (size_t)d->O * sizeof(float);

@@ -560,6 +560,25 @@ case("dot-view-strided-slice-of-argument", lambda b, x, y: b.matmul(b.slice(x, [
 case("dot-view-transpose-of-argument", lambda b, x, y: b.matmul(b.transpose(x, [1, 0]), b.transpose(y, [1, 0])), f32(2008, 70, 33), f32(2009, 45, 70))
 case("dot-view-reshape-merging-dims", lambda b, x, y: b.matmul(b.reshape(b.slice(x, [0, 0, 0], [4, 6, 35]), (24, 35)), y), f32(2010, 4, 6, 40), f32(2011, 35, 12))
 case("dot-view-reshape-not-a-view", lambda b, x, y: b.matmul(b.reshape(b.slice(x, [0, 0, 0], [4, 5, 35]), (20, 35)), y), f32(2012, 4, 6, 35), f32(2013, 35, 12))
+# the same at sizes past the small-product kernel: rows and columns of a slice are further apart than they are long, so the last ones lie
+# beyond rows x length of the view.  Contracted extents that are and are not a multiple of 16, every layout the vector loaders take
+# (contracted dim contiguous, rows or columns contiguous), a bias, a step between rows, a view that starts off a 16-byte boundary.
+def _sliced(b, x, r0, r1, c0, c1, step=1):
+    return b.slice(x, [r0, c0], [r1, c1], [step, 1])
+
+
+for _k in (500, 504, 512):
+    case(f"dot-view-large-lhs-columns-k{_k}", lambda b, x, y, _k=_k: b.matmul(_sliced(b, x, 0, 640, 0, _k), y), f32(2700 + _k, 640, 1024, lo=-0.1, hi=0.1), f32(2701 + _k, _k, 640, lo=-0.1, hi=0.1))
+    case(f"dot-view-large-lhs-columns-bias-k{_k}", lambda b, x, y, c, _k=_k: _linear(b, _sliced(b, x, 0, 640, 520, 520 + _k), y, c),
+         f32(2702 + _k, 640, 1040, lo=-0.1, hi=0.1), f32(2703 + _k, _k, 640, lo=-0.1, hi=0.1), f32(2704 + _k, 640, lo=-1, hi=1))
+    case(f"dot-view-large-rhs-columns-k{_k}", lambda b, x, y, _k=_k: b.matmul(x, _sliced(b, y, 0, _k, 640, 1280)), f32(2705 + _k, 640, _k, lo=-0.1, hi=0.1), f32(2706 + _k, _k, 1920, lo=-0.1, hi=0.1))
+    case(f"dot-view-large-both-k{_k}", lambda b, x, y, _k=_k: b.dot_general(_sliced(b, x, 0, 640, 0, _k), _sliced(b, y, 0, 640, 4, 4 + _k), ([1], [1])),
+         f32(2707 + _k, 640, 1024, lo=-0.1, hi=0.1), f32(2708 + _k, 640, 1032, lo=-0.1, hi=0.1))
+    case(f"dot-view-large-contracted-rows-k{_k}", lambda b, x, y, _k=_k: b.dot_general(_sliced(b, x, 0, _k, 0, 640), _sliced(b, y, 0, _k, 320, 960), ([0], [0])),
+         f32(2709 + _k, _k, 1280, lo=-0.1, hi=0.1), f32(2710 + _k, _k, 1280, lo=-0.1, hi=0.1))
+case("dot-view-large-every-other-row", lambda b, x, y: b.matmul(_sliced(b, x, 0, 1279, 0, 500, 2), y), f32(2720, 1279, 600, lo=-0.1, hi=0.1), f32(2721, 500, 640, lo=-0.1, hi=0.1))
+case("dot-view-large-odd-start", lambda b, x, y: b.matmul(_sliced(b, x, 0, 640, 3, 503), y), f32(2722, 640, 1024, lo=-0.1, hi=0.1), f32(2723, 500, 640, lo=-0.1, hi=0.1))
+case("dot-view-large-few-rows-long-k", lambda b, x, y: b.matmul(_sliced(b, x, 0, 96, 0, 4000), _sliced(b, y, 0, 4000, 0, 512)), f32(2724, 96, 4400, lo=-0.1, hi=0.1), f32(2725, 4000, 1024, lo=-0.1, hi=0.1))
 case("dot-view-same-buffer-twice", lambda b, x: b.dot_general(b.slice(x, [0, 0], [16, 40]), b.slice(x, [16, 0], [32, 40]), ([1], [1])), f32(2014, 32, 40))
 case("dot-int32-matmul", lambda b, x, y: b.matmul(x, y), i32(1930, 33, 70), i32(1931, 70, 45), exact=True)
 case("dot-int32-batched-attention-layout", lambda b, q, k: b.dot_general(q, k, ([3], [3]), ([0, 2], [0, 2])), i32(1932, 2, 9, 3, 16), i32(1933, 2, 11, 3, 16), exact=True)
