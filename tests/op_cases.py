@@ -714,6 +714,37 @@ case("softmax-rows-5000", _softmax_of, f32(2732, 7, 5000, lo=-6, hi=6))
 case("softmax-rows-bf16-768", _softmax_of, f32(2733, 24, 768, lo=-4, hi=4), dtypes=["bf16"])
 case("layer-norm-768-bf16", _layer_norm_of, f32(2734, 40, 768), f32(2735, 768), f32(2736, 768), dtypes=["bf16", "bf16", "bf16"])
 case("layer-norm-1536", _layer_norm_of, f32(2737, 12, 1536), f32(2738, 1536), f32(2739, 1536))
+# a division by one number per row: fewer than 256 rows divide (the same bits as the quotient of the two numbers); more multiply by a
+# reciprocal, which has to hold where the reciprocal itself is no normal number (sums below 2^-126 or from 2^126 on), zero, infinite or NaN
+def _divide_by_row(kind):
+    def f(b, x):
+        r = b.reduce_max(x, [1]) if kind == "max" else b.reduce_sum(x, [1])
+        return b.div(x, b.broadcast_in_dim(r, x.shape, [0]))
+    return f
+
+
+def _odd_rows(seed, *shape):
+    a = f32(seed, *shape, lo=0.1, hi=2)
+    a[0] = 0
+    a[0, :10] = 1e-40
+    a[1] = 0
+    a[2] *= 1e38 / shape[1]
+    a[3, 5] = np.inf
+    a[4, 7] = np.nan
+    a[5] = 0
+    a[5, 3], a[5, 4] = 3e-39, 1e-45
+    a[6] *= -1e-42
+    a[7] = 0
+    a[7, 0], a[7, 1], a[7, 2] = 2.0 ** 127, -(2.0 ** 126), 2.0 ** -100
+    a[8] = 0
+    a[8, 9] = -np.inf
+    return a
+
+
+for _rows in (9, 255, 256, 300):
+    case(f"rows-divide-by-sum-odd-values-{_rows}", _divide_by_row("sum"), _odd_rows(2750 + _rows, _rows, 200))
+for _rows, _cols in ((1, 4096), (9, 1000), (255, 130)):
+    case(f"rows-divide-by-maximum-exact-{_rows}", _divide_by_row("max"), f32(2751 + _rows, _rows, _cols, lo=0.1, hi=2), exact=True)
 # per-channel chains with a division and a square root that a large kernel reads through a broadcast: stored by the pass
 # that folds the sums they depend on, or by a kernel of their own when they depend on no reduction
 def _bn_like(b, x, g):
