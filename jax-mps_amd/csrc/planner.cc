@@ -313,6 +313,8 @@ class Planner {
     // is stored instead.
     std::unordered_map<Value*, int64_t> contexts;
     std::unordered_map<Value*, std::vector<Op*>> groups;
+    std::unordered_map<Op*, size_t> at;   // position in the region
+    for (size_t k = 0; k < r.ops.size(); ++k) at[r.ops[k].get()] = k;
     for (int k = (int)r.ops.size() - 1; k >= 0; --k) {
       Op* op = r.ops[k].get();
       if (!isFusibleOp(*op) || op->results.size() != 1) continue;
@@ -357,7 +359,7 @@ class Planner {
         for (auto* o : op->operands) if (o->def && !needMat_[o] && isExpensive(o->def->name) && o->def->parent == &r) expensive = true;
         // g consumers each re-reading `big` leaves move g*big tensors; materialising moves big + 1 + g and costs a launch
         static const int limit = getenv("MI355X_RECOMPUTE_LIMIT") ? atoi(getenv("MI355X_RECOMPUTE_LIMIT")) : 1;
-        if ((big >= 2 && ((int)g.size() - 1) * (big - 1) > limit && !readByOneRowProgram(v, g)) || expensive) mat = true;
+        if ((big >= 2 && ((int)g.size() - 1) * (big - 1) > limit && !readByOneRowProgram(v, r, at)) || expensive) mat = true;
       }
       contexts[v] = mat ? 1 : positions;
       needMat_[v] = mat;
@@ -726,6 +728,8 @@ class Planner {
     for (auto* o : v->def->operands) collectLeavesOf(o, out, seen);
   }
 
+  static constexpr size_t kRowProgramWindow = 96;   // ops after its first reduction that a row program looks at
+
   // Is this a reduction over the trailing dims with rows a row program takes?
   bool reducesWholeRows(const Op& op, std::vector<int64_t>& rd) {
     const TensorType& xt = op.operands[0]->type;
@@ -742,23 +746,88 @@ class Planner {
     return (Kn >= 256 || Rn <= 4096) && Rn >= 2 && Rn <= 32768;
   }
 
-  // Will one row program hold all readers of v?  Its first reduction and everything of v's shape that is computed from it:
-  // the kernel then evaluates v once per element and keeps it in registers, so there is nothing to gain from storing it
-  // (the sum a LayerNorm normalises: two reductions and the result read it).
-  bool readByOneRowProgram(Value* v, const std::vector<Op*>& readers) {
-    bool rows = false;
+  static bool rowProgramsOn() {
+    static const bool on = !(getenv("MI355X_ROW_PROGRAMS") && getenv("MI355X_ROW_PROGRAMS")[0] == '0');
+    return on;
+  }
+
+  // tensors a kernel that evaluates v would read, as far as that is known before the values above v are decided: a fusible value that
+  // a step needs in memory counts as one, and so does one with several readers (it is stored unless it reads one or two itself)
+  void likelyReads(Value* v, Region& r, std::unordered_set<Value*>& out, std::unordered_set<Value*>& seen, size_t limit) {
+    for (auto* o : v->def->operands) {
+      if (out.size() > limit || !seen.insert(o).second) continue;
+      bool memory = !o->def || o->def->parent != &r || !isFusibleOp(*o->def) || o->users.size() >= 2;
+      for (Op* u : o->users) if (u->parent != &r || forcedBy(o, u)) memory = true;
+      if (memory) out.insert(o);
+      else likelyReads(o, r, out, seen, limit);
+    }
+  }
+
+  // Will one row program hold every reader of v: reductions over its rows, and values of its shape that are stored, read v where
+  // they are evaluated themselves, and need nothing but those reductions and what is in memory ahead of the first of them (the sum
+  // a LayerNorm normalises: two reductions and the result read it)?  The kernel then evaluates v once per element and keeps it in
+  // registers, so there is nothing to gain from storing it.  A reader behind a product (the next sum of a residual stream that is
+  // normalised ahead of its layers) is not held: it would evaluate v again, and with it every earlier sum.
+  bool readByOneRowProgram(Value* v, Region& r, const std::unordered_map<Op*, size_t>& at) {
+    if (!rowProgramsOn()) return false;
+    // rows of at most eight walks are kept in registers between the walks (generateRowProgram); longer ones are read again by each
+    const int64_t last = v->type.dims.empty() ? 1 : v->type.dims.back();
+    const int64_t vec = last % 4 == 0 ? 4 : last % 2 == 0 ? 2 : 1;
+    std::vector<Op*> reduces, roots, todo{v->def};
+    std::unordered_set<Op*> seen;
     std::vector<int64_t> first, rd;
-    for (Op* u : readers) {
-      if (u->name == "reduce") {
-        if (!isSimpleReduce(*u) || u->operands[0]->type.dims != v->type.dims || !reducesWholeRows(*u, rd)) return false;
-        if (rows && rd != first) return false;
-        first = rd;
-        rows = true;
-      } else if (u->results.size() != 1 || !isFusibleOp(*u) || u->result()->type.dims != v->type.dims) {
-        return false;
+    while (!todo.empty()) {
+      Op* d = todo.back();
+      todo.pop_back();
+      for (Op* u : d->result()->users) {
+        if (u->parent != &r) return false;
+        if (!seen.insert(u).second) continue;
+        if (seen.size() > 64) return false;
+        if (u->name == "reduce") {
+          if (!isSimpleReduce(*u) || u->operands[0]->type.dims != v->type.dims || !reducesWholeRows(*u, rd)) return false;
+          if (!reduces.empty() && rd != first) return false;
+          first = rd;
+          reduces.push_back(u);
+        } else if (!sameShapeElementwise(*u) || u->result()->type.dims != v->type.dims) {
+          return false;
+        } else {
+          (needMat_[u->result()] ? roots : todo).push_back(u);
+        }
       }
     }
-    return rows;
+    if (reduces.empty() || reduces.size() > 4 || roots.size() > 8) return false;   // the program's own limits
+    int64_t rowElems = 1;
+    for (auto d : first) rowElems *= v->type.dims[(size_t)d];
+    if (rowElems > 2048 * vec) return false;
+    size_t begin = SIZE_MAX;
+    for (Op* u : reduces) begin = std::min(begin, at.at(u));
+    for (auto* list : {&reduces, &roots}) for (Op* u : *list) if (at.at(u) > begin + kRowProgramWindow) return false;
+    // what a member computes from: those reductions, or values from ahead of the first one
+    std::unordered_set<Value*> visited;
+    std::function<bool(Value*, bool&)> inside = [&](Value* x, bool& fromRows) -> bool {
+      Op* d = x->def;
+      auto p = d ? at.find(d) : at.end();
+      if (p == at.end() || p->second < begin) return true;
+      if (std::find(reduces.begin(), reduces.end(), d) != reduces.end()) { fromRows = true; return true; }
+      if (!isFusibleOp(*d) || d->results.size() != 1 || visited.size() > 256) return false;
+      if (!visited.insert(x).second) return true;
+      for (auto* o : d->operands) if (!inside(o, fromRows)) return false;
+      return true;
+    };
+    for (Op* u : reduces) {
+      bool fromRows = false;
+      visited.clear();
+      for (auto* o : u->operands) if (!inside(o, fromRows)) return false;
+    }
+    for (Op* u : roots) {
+      bool fromRows = false;
+      visited.clear();
+      if (!inside(u->result(), fromRows) || !fromRows) return false;
+    }
+    // a sum of many tensors goes through memory: its reductions may end up in kernels of their own (a kernel takes 60 arguments)
+    std::unordered_set<Value*> reads, below;
+    likelyReads(v, r, reads, below, 16);
+    return reads.size() <= 16;
   }
 
   // Softmax / LayerNorm shaped subgraphs: reductions over the trailing dims, elementwise values
@@ -766,8 +835,7 @@ class Planner {
   // in one kernel that owns whole rows (reference: the mps.softmax / mps.layer_norm custom calls
   // its fusion passes produce, passes/fuse_softmax.cc:174-247, passes/fuse_layer_norm.cc:229-354).
   bool tryRowProgram(Op* op, Region& r, size_t pos, Plan& plan) {
-    static const bool enabled = !(getenv("MI355X_ROW_PROGRAMS") && getenv("MI355X_ROW_PROGRAMS")[0] == '0');
-    if (!enabled || !isSimpleReduce(*op)) return false;
+    if (!rowProgramsOn() || !isSimpleReduce(*op)) return false;
     std::vector<int64_t> rd;
     if (!reducesWholeRows(*op, rd)) return false;
     const TensorType& xt = op->operands[0]->type;
@@ -790,8 +858,7 @@ class Planner {
       for (auto* o : d->operands) if (!can(o, dep, seen)) return false;
       return true;
     };
-    const size_t kWindow = 96;
-    for (size_t q = pos; q < r.ops.size() && q <= pos + kWindow; ++q) {
+    for (size_t q = pos; q < r.ops.size() && q <= pos + kRowProgramWindow; ++q) {
       Op* y = r.ops[q].get();
       if (emitted_.count(y)) continue;
       if (y->name == "reduce") {

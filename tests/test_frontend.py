@@ -195,6 +195,61 @@ def test_a_column_reduction_stores_the_value_it_reads_first():
     assert r.stdout.count("storing select") == 34 and "fusion:select" not in r.stdout        # 17 batch-norm backward passes, two launches each
 
 
+def _kernels(text):
+    """(label, bytes) of the plan's generated kernels and the number of distinct ones."""
+    r = plan(text, "--dump-plan")
+    assert r.returncode == 0, r.stderr
+    lines = [line for line in r.stdout.splitlines() if line.startswith("kernel ")]
+    return [(line.split(" k")[0], int(line.rsplit("bytes ", 1)[1].split()[0])) for line in lines], int(r.stdout.rsplit("steps, ", 1)[1].split()[0])
+
+
+def _residual_stack(layers, dtype, norm_first, rows=1024, d=768):
+    from jax_mps_amd.shlo.builder import Builder, layer_norm
+    b = Builder("residual_stack")
+    x, s, t, w1, w2 = (b.arg(shape, dtype) for shape in ((rows, d), (d,), (d,), (d, 2 * d), (2 * d, d)))
+    for _ in range(layers):
+        h = layer_norm(b, x, s, t, 1e-5) if norm_first else x
+        x = b.add(x, b.matmul(b.maximum(b.matmul(h, w1), 0.0), w2))
+        x = x if norm_first else layer_norm(b, x, s, t, 1e-5)
+    b.ret(layer_norm(b, x, s, t, 1e-5) if norm_first else x)
+    return b.text()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_a_stack_that_normalises_ahead_of_its_layers_moves_the_same_bytes_in_every_layer(dtype):
+    """A sum of the residual stream is read by its LayerNorm and, behind two products, by the next sum: it is stored, or every LayerNorm
+    would add up all earlier layers again."""
+    total = {n: _kernels(_residual_stack(n, dtype, True)) for n in (6, 12, 24)}
+    moved = {n: sum(nbytes for _, nbytes in kernels) for n, (kernels, _) in total.items()}
+    assert moved[24] - moved[12] <= 1.05 * 2 * (moved[12] - moved[6])
+    assert len(total[24][0]) - len(total[12][0]) == 2 * (len(total[12][0]) - len(total[6][0]))
+    assert total[24][1] <= total[6][1] + 1        # layers share their kernels
+
+
+def test_a_sum_that_one_row_program_reads_is_not_stored(monkeypatch):
+    """Normalised after the sum, it is computed inside the LayerNorm's kernel; where no row program will hold all of its readers (none are
+    made, rows too long for registers, a reader that moves data, a sum of very many tensors) it goes through memory."""
+    from jax_mps_amd.shlo.builder import Builder, layer_norm
+    adds = lambda kernels: sum(label.startswith("kernel fusion:add") for label, _ in kernels[0])   # noqa: E731
+    assert adds(_kernels(_residual_stack(3, "f32", False))) == 0
+    assert adds(_kernels(_residual_stack(3, "f32", False, rows=37))) == 0
+    assert adds(_kernels(_residual_stack(3, "f32", False, rows=300, d=16384))) == 3
+
+    def stack(count, mirrored=False):
+        b = Builder("sum_of_many")
+        xs = [b.arg((512, 256), "f32") for _ in range(count)]
+        s, t = b.arg((256,), "f32"), b.arg((256,), "f32")
+        y = xs[0]
+        for x in xs[1:]:
+            y = b.add(y, x)
+        out = layer_norm(b, y, s, t, 1e-5)
+        b.ret(out, *([b.mul(b.reverse(y, [1]), out)] if mirrored else []))
+        return _kernels(b.text())
+    assert adds(stack(3)) == 0 and adds(stack(40)) == 1 and adds(stack(3, mirrored=True)) == 1
+    monkeypatch.setenv("MI355X_ROW_PROGRAMS", "0")
+    assert adds(_kernels(_residual_stack(3, "f32", False))) == 6        # the sums, and what the LayerNorms return
+
+
 def test_location_aliases_result_lists_and_composites_parse():
     text = """#loc1 = loc("x")
 module @jit_f attributes {mhlo.num_partitions = 1 : i32} {
