@@ -607,13 +607,18 @@ static int launchFew(const mi355_gemm_desc* d, const void* a, const void* b, voi
   if (!rowsOfK && !kContiguous) return -1;
   if (d->batch0 > 1 && (d->aB0 % 8 || d->bB0 % 8)) return -1;
   if (d->batch1 > 1 && (d->aB1 % 8 || d->bB1 % 8)) return -1;
-  // While every workgroup of 64 rows has a compute unit of its own.  Measured against the 64x64 tiles of the ring kernel
-  // (K x N: us at the largest M inside the line, then at the next one): 768x768 7.5 / 8.4 at M = 512, 10.9 / 8.4 at 768;
-  // 3072x768 18.1 / 23.5 at 512, 33 / 23.5 at 768; 768x2304 7.6 / 8.3 at 192, 11.2 / 8.7 at 256; 768x3072 7.8 / 8.3 at 128,
-  // 10.9 / 8.6 at 192.
+  // One workgroup per compute unit, and of those splits the fewest rows per workgroup: a unit takes in about 15 bytes a cycle here, so
+  // what one of them has to read sets the time (37 rows, 3072x768: 13.7 us as one tile row of 48, 8.4 as three of 16).
+  // Measured against the 64x64 tiles of the ring kernel at 128 to 256 such units, both layouts of the rhs, products and batches of
+  // them, as its time over this kernel's: 32 rows 1.00 to 1.03 at K = 64, 1.00 to 1.16 at 256, 1.11 to 1.44 at 512, 1.35 to 1.69 at 768;
+  // 48 rows of [K][N] weights 1.01, 1.09, 1.09 and 1.26 upwards, of a k-contiguous rhs 0.99, 1.03, 0.93 and 1.16;
+  // 64 rows 0.84 to 0.90, 0.87 to 1.01, 0.79 to 0.94 and 0.99 to 1.15.  Two workgroups per unit lose (768x768 at 768 rows: 10.9 us to 8.4).
   constexpr long long kUnits = 256;
   const long long blocks = (d->M + 15) / 16, tilesN = (d->N + 31) / 32;
-  if ((blocks + 3) / 4 * tilesN * nb > kUnits) return -1;
+  const int most = d->K >= 768 ? 4 : rowsOfK ? 3 : 2;
+  int tmb = 1;
+  while (tmb <= most && (blocks + tmb - 1) / tmb * tilesN * nb > kUnits) ++tmb;
+  if (tmb > most) return -1;
   AsyncArgs g;
   g.a = (const u16*)a; g.b = (const u16*)b; g.c = c; g.bias = bias;
   g.M = d->M; g.N = d->N; g.K = d->K;
@@ -622,10 +627,6 @@ static int launchFew(const mi355_gemm_desc* d, const void* a, const void* b, voi
   g.batch1 = (int)d->batch1;
   g.outBf16 = d->out_dtype == 1;
   g.act = d->act; g.actA = d->act_a; g.actB = d->act_b; g.actC = d->act_c;
-  // the fewest rows per workgroup that still give each a unit of its own: a unit takes in about 15 bytes a cycle here, so what
-  // one of them has to read sets the time (37 rows, 3072x768: 13.7 us as one tile row of 48, 8.4 as three of 16)
-  int tmb = 1;
-  while ((blocks + tmb - 1) / tmb * tilesN * nb > kUnits) ++tmb;
   g.tilesM = (int)((blocks + tmb - 1) / tmb);
   g.tilesN = (int)tilesN;
   g.total = (long long)g.tilesM * g.tilesN * nb;

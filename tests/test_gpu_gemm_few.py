@@ -1,7 +1,7 @@
 """The bf16 product kernel for few output tiles (a workgroup per 16 to 64 rows and 32 columns, K shared out to its wavefronts):
 one row, ragged rows and columns, each number of row blocks, K of one slab, of fewer slabs than wavefronts, of a slab count
 that does not divide and of many slabs, both layouts of the right-hand side, bias, float32 results, a batch dim, and the
-largest grid it takes next to the first it leaves to the ring kernel."""
+largest grids it takes next to the first it leaves to the ring kernel (64 rows a workgroup from K = 768 on)."""
 import numpy as np
 import pytest
 
@@ -21,6 +21,16 @@ CASES = [
     ("two-blocks", (95, 160), (160, 2056), NN, ((), ()), False, "bf16"),
     ("three-blocks", (96, 64), (64, 4096), NN, ((), ()), True, "bf16"),
     ("four-blocks-largest", (64, 96), (96, 8192), NN, ((), ()), False, "bf16"),
+    # four and more slabs of K per wavefront, with remainders, for each number of row blocks and both layouts
+    ("two-blocks-long-k", (37, 800), (800, 3072), NN, ((), ()), True, "bf16"),
+    ("three-blocks-long-k", (96, 864), (864, 4096), NN, ((), ()), True, "bf16"),
+    ("four-blocks-long-k", (64, 928), (928, 8192), NN, ((), ()), True, "bf16"),
+    ("two-blocks-long-k-nt", (37, 832), (3072, 832), NT, ((), ()), True, "bf16"),
+    ("three-blocks-long-k-nt", (96, 896), (4090, 896), NT, ((), ()), False, "bf16"),
+    ("four-blocks-long-k-nt", (63, 800), (8192, 800), NT, ((), ()), True, "f32"),
+    ("four-blocks-short-k", (64, 736), (736, 8192), NN, ((), ()), True, "bf16"),
+    ("three-blocks-nt-short-k", (96, 512), (4096, 512), NT, ((), ()), False, "bf16"),
+    ("three-blocks-nt", (96, 768), (4096, 768), NT, ((), ()), False, "bf16"),
     ("past-the-line", (65, 128), (128, 8192), NN, ((), ()), False, "bf16"),
     ("nt-odd-columns", (33, 224), (33, 224), NT, ((), ()), False, "bf16"),
     ("nt-f32-odd-columns", (50, 192), (45, 192), NT, ((), ()), True, "f32"),
