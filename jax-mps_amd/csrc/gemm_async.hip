@@ -642,8 +642,10 @@ static int launchFew(const mi355_gemm_desc* d, const void* a, const void* b, voi
 extern "C" int mi355_gemm_bf16_async(const mi355_gemm_desc* d, const void* a, const void* b, void* c, const void* bias, void* workspace,
                                      size_t workspace_bytes, mi355_stream_t s) {
   static const char* force = getenv("MI355X_GEMM_TILE");   // "256x128", "128x128", "128x64", "64x64": tuning aid
-  const int wideMode = getenv("MI355X_GEMM_WIDE") ? atoi(getenv("MI355X_GEMM_WIDE")) : 1;   // read at every call: tests switch it
-  if (!force && wideMode == 1)                             // (a forced tiling is one of the ring kernel's)
+  const int wideMode = getenv("MI355X_GEMM_WIDE") ? atoi(getenv("MI355X_GEMM_WIDE")) : 1;   // both read at every call: tests switch them
+  const bool fewOn = !getenv("MI355X_GEMM_FEW") || atoi(getenv("MI355X_GEMM_FEW")) != 0;
+  const bool wideForced = wideMode == 2 && d->M >= 256 && d->N >= 256;
+  if (!force && fewOn && !wideForced)                      // (a forced tiling is one of the ring kernel's)
     if (const int few = launchFew(d, a, b, c, bias, (hipStream_t)s); few >= 0) return few;
   OperandPlan pa, pb;
   if (!qualifies(d, pa, pb)) return -1;

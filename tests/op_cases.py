@@ -383,6 +383,7 @@ case("dot-bf16-async-nt-big", lambda b, x, y: b.dot_general(x, y, ([1], [1])), f
 def i32(seed, *shape, lo=-1000, hi=1000):
     return rng(seed).integers(lo, hi, size=shape).astype(np.int32)
 # n-contiguous rhs (a dense layer's [in, out] weights) read in place by the LDS-ring kernel, one case per tile shape
+# (the small ones by the kernel for few output tiles; tests/test_gpu_gemm_few.py runs them on the ring kernel too)
 case("dot-bf16-async-nn-edges", lambda b, x, y: b.matmul(x, y), f32(1950, 200, 128, lo=-1, hi=1), f32(1951, 128, 328, lo=-1, hi=1), dtypes=["bf16", "bf16"])
 case("dot-bf16-async-nn-narrow", lambda b, x, y: b.matmul(x, y), f32(1952, 300, 64, lo=-1, hi=1), f32(1953, 64, 72, lo=-1, hi=1), dtypes=["bf16", "bf16"])
 case("dot-bf16-async-nn-batched", lambda b, x, y: b.dot_general(x, y, ([2], [1]), ([0], [0])), f32(1954, 3, 130, 64, lo=-1, hi=1), f32(1955, 3, 64, 136, lo=-1, hi=1), dtypes=["bf16", "bf16"])
