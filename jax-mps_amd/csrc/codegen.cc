@@ -1539,9 +1539,10 @@ FusedCode generateReduceKernel(const std::vector<Op*>& reduces, const LeafPredic
   int TY = 256 / TX;
   int64_t gridX = (kvecs + TX - 1) / TX;
   int64_t P = 1;
-  // Sixteen visits per lane are best while that gives workgroups for half the compute units (64 of them: ResNet18's statistics at
-  // batch 16, one wavefront per SIMD walking sixteen dependent-latency loads; its forward pass 559 us with sixteen visits,
-  // 551 with eight, and at batch 128, 512 workgroups, the train step 4716 us with sixteen and 4763 with eight).
+  // Sixteen visits per lane, dependent in their latency, where that gives workgroups for half of the compute units, eight where it does
+  // not (ResNet18's statistics at batch 16 are 64 workgroups or fewer, at batch 128 those of its 512 channels).  Measured with sixteen,
+  // this rule and eight everywhere: forward pass at batch 16 567, 555 and 557 us, train step at batch 128 4737, 4735 and 4772;
+  // sum and sum of squares of 50000 x 24 alone 8.9 us with sixteen and 7.9 with eight.
   static const int colEnv = getenv("MI355X_REDUCE_COL_PER_THREAD") ? atoi(getenv("MI355X_REDUCE_COL_PER_THREAD")) : 0;
   const int colPerThread = colEnv ? colEnv : ((Rn + TY * 16 - 1) / (TY * 16) * gridX < 128 ? 8 : 16);
   if (Rn > (int64_t)TY * 16) P = std::min<int64_t>((Rn + TY * colPerThread - 1) / (TY * colPerThread), std::max<int64_t>(1, 2048 / gridX));

@@ -398,6 +398,11 @@ def _linear(b, x, w, bias):
 
 case("dot-bias-f32-small", _linear, f32(1970, 33, 70), f32(1971, 70, 45), f32(1972, 45))
 case("dot-bias-f32-igemm", _linear, f32(1973, 520, 384, lo=-1, hi=1), f32(1974, 384, 1030, lo=-1, hi=1), f32(1975, 1030))
+# a bias added by the stores themselves: 16-byte and single stores of an unsplit product, the fold of a few and of many K ranges
+case("dot-bias-f32-igemm-unsplit-vector-stores", _linear, f32(2680, 2050, 100, lo=-1, hi=1), f32(2681, 100, 1536, lo=-1, hi=1), f32(2682, 1536))
+case("dot-bias-f32-igemm-unsplit-single-stores", _linear, f32(2683, 2050, 100, lo=-1, hi=1), f32(2684, 100, 1030, lo=-1, hi=1), f32(2685, 1030))
+case("dot-bias-f32-igemm-fold-of-three", _linear, f32(2686, 520, 384, lo=-1, hi=1), f32(2687, 384, 1032, lo=-1, hi=1), f32(2688, 1032))
+case("dot-bias-f32-igemm-fold-of-many", _linear, f32(2689, 130, 9600, lo=-0.1, hi=0.1), f32(2690, 9600, 132, lo=-0.1, hi=0.1), f32(2691, 132))
 case("dot-bias-f32-3d", _linear, f32(1976, 4, 9, 70), f32(1977, 70, 24), f32(1978, 24))
 case("dot-bias-bf16-async", _linear, f32(1979, 200, 128, lo=-1, hi=1), f32(1980, 128, 328, lo=-1, hi=1), f32(1981, 328), dtypes=["bf16", "bf16", "bf16"])
 case("dot-bias-bf16-tiled", _linear, f32(1982, 200, 136, lo=-1, hi=1), f32(1983, 136, 328, lo=-1, hi=1), f32(1984, 328), dtypes=["bf16", "bf16", "bf16"])
@@ -673,6 +678,8 @@ def _conv_stats(padding=((1, 1), (1, 1)), kind="add"):
 case("conv-statistics-from-accumulators", _conv_stats(), f32(1320, 24, 32, 32, 16, lo=0.05, hi=1.0), f32(1321, 3, 3, 16, 64, lo=0.05, hi=1.0))
 case("conv-statistics-ragged-rows-two-feature-tiles", _conv_stats(), f32(1322, 12, 31, 31, 16, lo=0.05, hi=1.0), f32(1323, 3, 3, 16, 128, lo=0.05, hi=1.0))
 case("conv-statistics-100-features", _conv_stats(), f32(1324, 12, 31, 31, 16, lo=0.05, hi=1.0), f32(1325, 3, 3, 16, 100, lo=0.05, hi=1.0))
+case("conv-statistics-24-features-in", _conv_stats(), f32(1332, 24, 32, 32, 24, lo=0.05, hi=1.0), f32(1333, 3, 3, 24, 64, lo=0.05, hi=1.0))
+case("conv-statistics-20-features-in-ragged-rows", _conv_stats(), f32(1334, 12, 31, 31, 20, lo=0.05, hi=1.0), f32(1335, 3, 3, 20, 100, lo=0.05, hi=1.0))
 case("conv-statistics-split-k-stays-unfused", _conv_stats(), f32(1326, 2, 4, 4, 256, lo=0.05, hi=1.0), f32(1327, 3, 3, 256, 64, lo=0.05, hi=1.0))
 case("conv-statistics-max-stays-unfused", _conv_stats(kind="max"), f32(1328, 24, 32, 32, 16, lo=0.05, hi=1.0), f32(1329, 3, 3, 16, 64, lo=0.05, hi=1.0))
 case("conv-bf16", _conv(padding=((1, 1), (1, 1))), u(240, 2, 8, 8, 16), u(241, 3, 3, 16, 8), dtypes=["bf16", "bf16"])
@@ -691,6 +698,9 @@ case("reduce-sum-int", lambda b, x: b.reduce_sum(x, [0]), i32(259, 100, 7), exac
 case("reduce-and-or", lambda b, x: [b._reduce(x, [1], "and", True), b._reduce(x, [1], "or", False)], rng(260).integers(0, 2, size=(6, 9)).astype(bool), exact=True)
 case("reduce-long-row", lambda b, x: b.reduce_sum(x, [1]), f32(261, 3, 70000, lo=-1, hi=1))
 case("reduce-tall-column", lambda b, x: b.reduce_sum(x, [0]), f32(262, 50000, 24, lo=-1, hi=1))
+# the largest column reduction of 24 columns whose lanes make eight visits, and the smallest whose lanes make sixteen
+for _rows in (65024, 65025):
+    case(f"reduce-tall-columns-{_rows}", lambda b, x: [b.reduce_sum(x, [0]), b.reduce_sum(b.mul(x, x), [0])], f32(2630 + _rows, _rows, 24, lo=-1, hi=1))
 case("reduce-full-large", lambda b, x: b.reduce_sum(x, [0]), f32(263, 1 << 20, lo=-1, hi=1))
 case("reduce-siblings", lambda b, x: [b.reduce_sum(x, [0, 1, 2]), b.reduce_sum(b.mul(x, x), [0, 1, 2])], f32(264, 8, 12, 12, 32))
 case("reduce-fused-input", lambda b, x, m: b.reduce_sum(b.mul(b.sub(x, b.broadcast_in_dim(m, x.shape, [1])), 2.0), [0]), f32(265, 300, 40), f32(266, 40))
@@ -746,6 +756,24 @@ for _rows in (9, 255, 256, 300):
     case(f"rows-divide-by-sum-odd-values-{_rows}", _divide_by_row("sum"), _odd_rows(2750 + _rows, _rows, 200))
 for _rows, _cols in ((1, 4096), (9, 1000), (255, 130)):
     case(f"rows-divide-by-maximum-exact-{_rows}", _divide_by_row("max"), f32(2751 + _rows, _rows, _cols, lo=0.1, hi=2), exact=True)
+# the shortest and longest rows that fewer than 256 of them run as a row program, and the first longer one
+for _rows, _cols in ((1, 2), (1, 4096), (255, 4096), (1, 4097), (3, 4100)):
+    case(f"softmax-few-rows-{_rows}x{_cols}", _softmax_of, f32(2760 + _rows + _cols, _rows, _cols, lo=-6, hi=6))
+    case(f"layer-norm-few-rows-{_rows}x{_cols}", _layer_norm_of, f32(2761 + _rows + _cols, _rows, _cols), f32(2762 + _cols, _cols), f32(2763 + _cols, _cols))
+case("softmax-few-rows-two-trailing-dims", lambda b, x: (lambda e: b.div(e, b.broadcast_in_dim(b.reduce_sum(e, [1, 2]), x.shape, [0])))(b.exp(x)), f32(2764, 5, 24, 40, lo=-3, hi=3))
+
+
+def _special_rows(seed, *shape):
+    a = f32(seed, *shape, lo=-6, hi=6)
+    a[0, 3] = np.inf
+    a[1, 4] = np.nan
+    a[2] = -np.inf
+    a[3, 1:] = -np.inf
+    a[4] = np.finfo(np.float32).min
+    return a
+case("softmax-few-rows-special-values", _softmax_of, _special_rows(2765, 11, 300))
+case("softmax-many-rows-special-values", _softmax_of, _special_rows(2766, 260, 300))
+
 # per-channel chains with a division and a square root that a large kernel reads through a broadcast: stored by the pass
 # that folds the sums they depend on, or by a kernel of their own when they depend on no reduction
 def _bn_like(b, x, g):

@@ -309,12 +309,19 @@ module @jit_f attributes {jax.uses_shape_polymorphism = false, mhlo.num_partitio
     assert np.array_equal(got[0], np.array([16.5, 33.0, 49.5], np.float32)) and np.array_equal(got[1], [True, False]) and np.array_equal(got[2], [[1.0, 2.0]])
 
 
+def test_column_reductions_of_few_workgroups_make_eight_visits_a_lane():
+    grids = [plan(op_cases.get_case(f"reduce-tall-columns-{rows}").text, "--dump-plan").stdout.split(" grid ", 1)[1].split()[0] for rows in (65024, 65025)]
+    assert grids == ["1x254", "1x128"]        # 32 row lanes a workgroup: 127 workgroups of sixteen visits would be less than half of the compute units
+
+
 def test_convolution_delivers_batch_norm_statistics():
     """The column sum and sum of squares of an unsplit convolution's output come from its accumulators: the pass over
     the output is gone and only the fold of the per-tile sums remains; a convolution that splits K, or a reduction
     of another kind, keeps its own pass over the output."""
     r = plan(op_cases.get_case("conv-statistics-from-accumulators").text, "--dump-plan")
     assert "+ column statistics" in r.stdout and r.stdout.count("kernel ") == 1 and "fold of convolution statistics" in r.stdout
+    r = plan(op_cases.get_case("conv-statistics-24-features-in").text, "--dump-plan")        # contracted features that do not fill k-tiles of 16
+    assert "+ column statistics" in r.stdout
     r = plan(op_cases.get_case("conv-statistics-split-k-stays-unfused").text, "--dump-plan")
     assert "column statistics" not in r.stdout and "reduce" in r.stdout      # (small enough for single-pass reductions, which share a launch)
     r = plan(op_cases.get_case("conv-statistics-max-stays-unfused").text, "--dump-plan")
