@@ -114,7 +114,7 @@ __device__ __forceinline__ void storeAccumulators(const ConvP& p, float16v (&acc
   const bool partial = p.splitK > 1;
   const bool vec = p.outVec != 0;
   // The bias goes into the accumulators ahead of the stores.  Added to each value as it was stored it cost the convolutions, which have
-  // none, up to 6 % (8x16x16 images, 16 channels: 9.1 us without the code, 9.6 in the stores, 9.3 here) and the kernels a third more registers.
+  // none, up to 6 % (8x16x16 images, 16 channels: 9.1 us without the code, 9.6 in the stores, 9.3 here).
   if (p.bias && !partial) {
 #pragma unroll
     for (int b = 0; b < TN; ++b) {
