@@ -136,7 +136,8 @@ __global__ void __launch_bounds__(256) gemm_f32_mfma(GemmArgs g) {
   const long long b0 = blockIdx.z / g.batch1, b1 = blockIdx.z % g.batch1;
   const float* A = (const float*)g.a + b0 * g.aB0 + b1 * g.aB1;
   const float* B = (const float*)g.b + b0 * g.bB0 + b1 * g.bB1;
-  const long long m0 = (long long)blockIdx.y * BM, n0 = (long long)blockIdx.x * BN;
+  const unsigned tilesN = (unsigned)((g.N + BN - 1) / BN);
+  const long long m0 = (long long)(blockIdx.x / tilesN) * BM, n0 = (long long)(blockIdx.x % tilesN) * BN;
   float16v acc = {0};
   const bool aKfast = g.aCol == 1 || g.aRow != 1;   // walk k fastest when k is the contiguous axis
   const bool bNfast = g.bCol == 1 || g.bRow != 1;
@@ -363,7 +364,8 @@ __global__ void __launch_bounds__(256) gemm_bf16_mfma(GemmArgs g) {
   const long long b0 = blockIdx.z / g.batch1, b1 = blockIdx.z % g.batch1;
   const u16* A = (const u16*)g.a + b0 * g.aB0 + b1 * g.aB1;
   const u16* B = (const u16*)g.b + b0 * g.bB0 + b1 * g.bB1;
-  const long long m0 = (long long)blockIdx.y * BM, n0 = (long long)blockIdx.x * BN;
+  const unsigned tilesN = (unsigned)((g.N + BN - 1) / BN);
+  const long long m0 = (long long)(blockIdx.x / tilesN) * BM, n0 = (long long)(blockIdx.x % tilesN) * BN;
   float16v acc = {0};
   const bool aKfast = g.aCol == 1 || g.aRow != 1;
   const bool bNfast = g.bCol == 1 || g.bRow != 1;
@@ -1224,12 +1226,15 @@ int mi355_gemm(const mi355_gemm_desc* d, const void* a, const void* b, void* c, 
   mi355_conv_desc cd;
   // strided views may start anywhere; the implicit-GEMM loaders issue 16-byte loads
   if (gemmAsPointwiseConv(d, &cd) && (((uintptr_t)a | (uintptr_t)b) & 15) == 0) {
-    // the bias rides in the stores (or in the fold of a split K): the pass that added it took 4.5 to 7 us per layer
+    // the bias rides in the accumulators (or in the fold of a split K): the pass that added it took 4.5 to 7 us per layer
     // of 1024 rows, a tenth of the products' time
     return mi355_conv_bias(&cd, a, b, c, bias, workspace, workspace_bytes, s);
   }
   if (nb > 65535) return 1;   // grid.z limit; callers fold larger batches
-  dim3 grid((unsigned)((d->N + 63) / 64), (unsigned)((d->M + 63) / 64), (unsigned)nb);
+  // output tiles along x, columns fastest: y ends at 65535, which four million rows reach
+  const long long tiles = ((d->N + 63) / 64) * ((d->M + 63) / 64);
+  if (tiles > 0x7FFFFFFFll) return 1;
+  dim3 grid((unsigned)tiles, 1, (unsigned)nb);
   if (d->in_dtype == 0) gemm_f32_mfma<<<grid, 256, 0, (hipStream_t)s>>>(g);
   else if (d->in_dtype == 1) gemm_bf16_mfma<<<grid, 256, 0, (hipStream_t)s>>>(g);
   else return 2;
