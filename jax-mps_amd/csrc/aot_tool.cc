@@ -41,10 +41,14 @@ int main(int argc, char** argv) {
       if (dumpPlan) fputs(prog->dump.c_str(), stdout);
       if (dumpKernels)
         for (size_t k = 0; k < prog->kernels.size(); ++k) printf("// ===== kernel %zu =====\n%s\n", k, prog->kernels[k].source.c_str());
+      if (dumpPlan && prog->loopsAsKernels && atoi(getenv("MI355X_DUMP_PLAN")) >= 3) printf("// ===== with loops as kernels\n%s", prog->loopsAsKernels->dump.c_str());
+      if (dumpKernels && prog->loopsAsKernels)
+        for (auto& k : prog->loopsAsKernels->kernels) printf("// ===== kernel with loops as kernels\n%s\n", k.source.c_str());
       int disk = 0, comp = 0;
       if (compile) {
         std::vector<const std::string*> srcs;
         for (auto& k : prog->kernels) srcs.push_back(&k.source);
+        if (prog->loopsAsKernels) for (auto& k : prog->loopsAsKernels->kernels) srcs.push_back(&k.source);
         mi355::compileKernelSources(srcs, "gfx950", &disk, &comp);
       }
       printf("%s: %d ops -> %d steps, %zu fused kernels (%d compiled, %d cached), arena %.2f MiB, consts %zu B\n", a.c_str(),

@@ -75,6 +75,31 @@ FusedCode generateDusKernel(Op* dus, const LeafPredicate& isLeaf);
 int64_t sortLdsBytes(Op* sort);
 FusedCode generateSortKernel(Op* sort, const LeafPredicate& isLeaf);
 
+// A counted loop that recurrence.cc has matched, and the kernel that runs all its iterations (codegen.cc).
+struct Recurrence {
+  enum Kind { Counter, Passed, State, Stack, Accumulator };
+  Op* loop = nullptr;
+  int64_t trip = 0, counterInit = 0, counterStep = 0;
+  int counter = -1;
+  int64_t rows = 0, width = 0;            // carried states are float32 [rows, width]
+  Op* dot = nullptr;                      // [rows, contracted * width] . constant weights -> [rows, pieces * width]
+  int64_t pieces = 0, contracted = 0;
+  Value* weights = nullptr;
+  int64_t weightK = 0, weightN = 0;       // element strides of the weights along the contracted and the result dim
+  std::vector<Kind> kinds;                // per carry
+  struct Stacked { int carry = -1; Value* value = nullptr; int64_t base = 0, step = 0; bool covers = false; };
+  std::vector<Stacked> stacks;            // [.., rows, m * width] written at element base + step * iteration
+};
+struct RecurrenceCode {
+  std::string source;
+  unsigned blocks = 1;                    // of 256 lanes
+  std::vector<Value*> leaves;             // arguments in0, in1, ...; then init, final per state; then the stacks; exchange; flags, twice
+  int64_t exchangeBytes = 0, flagBytes = 0;
+};
+RecurrenceCode generateRecurrence(const Recurrence& r);   // throws CompileError: the loop holds something it has no form for
+// element offset of a window of `type` whose start indices are operands first, first + 1, ... of `op`, as base + step * iteration
+bool recurrenceOffset(const Recurrence& r, const Op& op, size_t first, const TensorType& type, const std::vector<int64_t>& sizes, int64_t& base, int64_t& step);
+
 // Several independent kernels with one-dimensional grids as the segments of one launch: block b
 // runs the kernel whose block range holds b.  Arguments are the kernels' arguments, concatenated.
 // Returns "" when one of the sources cannot take part (batchableKernel is the cheap test).

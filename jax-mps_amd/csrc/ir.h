@@ -63,6 +63,7 @@ struct Attr {
 
 struct Op;
 struct Region;
+struct RecurrenceOp;   // recurrence.h
 
 struct Value {
   int id = -1;
@@ -114,6 +115,7 @@ struct Op {
   }
   Value* result(int i = 0) const { return results[i].get(); }
   ConvDims convDims;  // for "convolution"
+  std::shared_ptr<RecurrenceOp> recurrence;  // for "recurrence" (a loop that runs as one kernel; no StableHLO op)
 };
 
 struct Func {
@@ -175,6 +177,10 @@ int64_t staticTripCount(Op* whileOp, LoopCounter* counter = nullptr);
 // inside counted loops, a product of a loop-invariant operand with the counter-selected slice of a loop-invariant tensor
 // becomes one product over the whole tensor ahead of the loop, and the body slices its result
 void hoistLoopProducts(Module& m);
+// counted loops chained through one float32 product and otherwise elementwise become "recurrence" ops, one kernel each, and what they
+// only accumulate becomes one product or sum behind them (recurrence.cc); false: there is no such loop
+bool lowerRecurrences(Module& m);
+std::unique_ptr<Module> cloneMain(const Module& m);   // a module of its own that holds a copy of main
 // updates = select(index in range, u, 0) ahead of a whole-row scatter with that index: the scatter reads u (rows out of
 // range are dropped by the scatter itself)
 void dropScatterIndexMasks(Module& m);

@@ -1665,6 +1665,55 @@ void rebuildUses(Region& r) {
   fill(r);
 }
 
+static void cloneRegion(const Region& from, Region& to, std::unordered_map<const Value*, Value*>& values) {
+  auto copyValue = [&](const Value& v) {
+    auto c = std::make_unique<Value>(v);
+    c->users.clear();
+    values[&v] = c.get();
+    return c;
+  };
+  for (auto& a : from.args) {
+    to.args.push_back(copyValue(*a));
+    to.args.back()->argOf = &to;
+  }
+  for (auto& o : from.ops) {
+    auto c = std::make_unique<Op>();
+    c->name = o->name;
+    c->attrs = o->attrs;
+    c->parent = &to;
+    c->line = o->line;
+    c->dead = o->dead;
+    c->convDims = o->convDims;
+    for (auto* v : o->operands) c->operands.push_back(values.at(v));
+    for (auto& sub : o->regions) {
+      c->regions.push_back(std::make_unique<Region>());
+      c->regions.back()->parent = c.get();
+      cloneRegion(*sub, *c->regions.back(), values);
+    }
+    for (auto& v : o->results) {
+      c->results.push_back(copyValue(*v));
+      c->results.back()->def = c.get();
+    }
+    to.ops.push_back(std::move(c));
+  }
+}
+
+std::unique_ptr<Module> cloneMain(const Module& m) {
+  const Func* from = m.main();
+  auto out = std::make_unique<Module>();
+  out->numPartitions = m.numPartitions;
+  out->numReplicas = m.numReplicas;
+  auto f = std::make_unique<Func>();
+  f->name = from->name;
+  f->isPublic = from->isPublic;
+  f->resultTypes = from->resultTypes;
+  f->argDonation = from->argDonation;
+  std::unordered_map<const Value*, Value*> values;
+  cloneRegion(from->body, f->body, values);
+  out->funcs.push_back(std::move(f));
+  return out;
+}
+
 int countOps(const Region& r) {
   int n = 0;
   for (auto& o : r.ops) {

@@ -158,6 +158,8 @@ struct CompiledProgram {
   std::vector<OutputInfo> outputs;
   std::vector<uint8_t> constPool;   // host image of the constant pool
   std::vector<std::vector<int64_t>> ivTables;   // per-iteration byte offsets of references that follow a host-side loop counter
+  // the same program with loops as kernels whose workgroups wait for each other (recurrence.cc), where it has such loops
+  std::unique_ptr<CompiledProgram> loopsAsKernels;
   int64_t arenaBytes = 0;
   int numOps = 0, numSteps = 0;
   std::string dump;                 // human-readable plan (MI355X_DUMP_PLAN)

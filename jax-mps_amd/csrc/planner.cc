@@ -22,6 +22,7 @@
 #include "codegen.h"
 #include "hip_abi.h"
 #include "plan.h"
+#include "recurrence.h"
 
 namespace mi355 {
 
@@ -534,6 +535,7 @@ class Planner {
       if (n == "scatter") { emitScatter(op, plan); return; }
       if (n == "sort") { emitSort(op, plan); return; }
       if (n == "dynamic_update_slice") { emitDus(op, plan); return; }
+      if (n == "recurrence") { emitRecurrence(op, plan); return; }
       if (n == "while") { emitWhile(op, plan); return; }
       if (n == "case") { emitCase(op, plan); return; }
       throw CompileError("no lowering for stablehlo." + n);
@@ -2533,6 +2535,49 @@ class Planner {
     plan.steps.push_back(std::move(w));
   }
 
+  // A loop that runs as one kernel (recurrence.cc): its flags are cleared, then one launch.
+  void emitRecurrence(Op* op, Plan& plan) {
+    const RecurrenceOp& rec = *op->recurrence;
+    for (auto* v : op->operands) if (!hasStorage(v)) materializeNow(v, plan);
+    const size_t leaves = rec.code.leaves.size();
+    std::vector<int> results;
+    for (size_t k = 0; k < op->results.size(); ++k) {
+      Value* v = op->results[k].get();
+      results.push_back(newStorage(v->type.bytes()));
+      const int init = k < rec.states ? -1 : rec.stackInit[k - rec.states];
+      if (init >= 0) copyStep(plan, storageOf(op->operands[(size_t)init]), results[k], (int64_t)v->type.bytes(), "recurrence stack init");
+    }
+    const int64_t zeros = ((int64_t)P.constPool.size() + kAlign - 1) / kAlign * kAlign;
+    P.constPool.resize((size_t)(zeros + rec.code.flagBytes), 0);
+    const int cleared = newStorage((size_t)rec.code.flagBytes, BufRef::Const), flags = newStorage((size_t)rec.code.flagBytes);
+    st_[cleared].offset = zeros;
+    copyStep(plan, cleared, flags, rec.code.flagBytes, "recurrence flags");
+    const int exchange = newStorage((size_t)rec.code.exchangeBytes);
+    const int t = ++time_;
+    Step s;
+    s.kind = Step::Kernel;
+    s.label = rec.label;
+    s.kernel = kernelId(rec.code.source);
+    s.grid[0] = rec.code.blocks;
+    s.block[0] = 256;
+    s.time = t;
+    auto arg = [&](int sid, bool writes) {
+      s.args.push_back(ref(sid, t));
+      s.argWrites.push_back(writes);
+    };
+    for (size_t k = 0; k < leaves; ++k) arg(storageOf(op->operands[k]), false);
+    for (size_t k = 0; k < rec.states; ++k) {
+      arg(storageOf(op->operands[leaves + k]), false);
+      arg(results[k], true);
+    }
+    for (size_t k = rec.states; k < results.size(); ++k) arg(results[k], true);
+    arg(exchange, true);
+    arg(flags, true);
+    arg(flags, false);   // (a kernel that writes what it reads is launched once where launches are repeated to be timed)
+    for (size_t k = 0; k < results.size(); ++k) bind(op->results[k].get(), results[k]);
+    plan.steps.push_back(std::move(s));
+  }
+
   void emitCase(Op* op, Plan& plan) {
     Value* index = op->operands[0];
     if (!hasStorage(index)) materializeNow(index, plan);
@@ -2978,6 +3023,19 @@ std::unique_ptr<CompiledProgram> compileProgram(std::unique_ptr<Module> module) 
   reluMasksFromActivations(*module);
   checkSupported(*module);
   eliminateDeadCode(module->main()->body);
+  bool loops = false;
+  for (auto& op : module->main()->body.ops) if (op->name == "while") loops = true;
+  if (loops) {
+    auto copy = cloneMain(*module);
+    if (lowerRecurrences(*copy)) {
+      eliminateDeadCode(copy->main()->body);
+      prog->loopsAsKernels = std::make_unique<CompiledProgram>();
+      prog->loopsAsKernels->paramDonation = prog->paramDonation;
+      prog->loopsAsKernels->module = std::move(copy);
+      Planner planner(*prog->loopsAsKernels);
+      planner.run();
+    }
+  }
   prog->module = std::move(module);
   Planner planner(*prog);
   planner.run();

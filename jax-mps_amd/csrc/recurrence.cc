@@ -1,0 +1,479 @@
+// Loops that run as one kernel.
+//
+// The loop of a recurrent network (jax.lax.scan lowers to stablehlo.while, reference: ops/control_flow.cc:702-989), once the
+// products that do not depend on what it carries have left it, is a chain: one product of the carried state with constant
+// weights per iteration, and elementwise work around it.  Run launch by launch an iteration costs two dependent launches,
+// and each product fetches the weights again.  Such a loop becomes one "recurrence" op, one kernel for all iterations
+// (codegen.cc, generateRecurrence).  What the loop's backward form only accumulates (weight gradients x[i]^T . g, bias
+// gradients, sums over the rows) does not belong to the chain: the rows g of all iterations are stacked and the
+// accumulation is one product, or sum, over the stack behind the loop.
+//
+// The workgroups of that kernel wait for each other, so all of them must fit the device at once.  A program with such loops
+// is therefore planned twice: as it is, and with them as kernels; the executable takes the second on a device that is
+// large enough (runtime.cc).
+#include "recurrence.h"
+
+#include <algorithm>
+#include <cstdlib>
+#include <functional>
+#include <unordered_set>
+
+namespace mi355 {
+
+namespace {
+
+constexpr int64_t kRecurrenceBlocks = 128;          // all run at once: at most one per two compute units
+constexpr int64_t kRecurrenceWeights = 128;         // registers a lane may hold of the weights
+constexpr int64_t kRecurrenceTrips = 8;             // shorter loops are left to their launches
+constexpr int64_t kStackBytes = (int64_t)256 << 20; // of one stack that an accumulation is taken over
+
+Region* regionOf(const Value* v) { return v->def ? v->def->parent : v->argOf; }
+
+// the value of the integer scalar `v` of `body` while the loop's counter holds `c`
+bool indexAt(Value* v, const Value* counter, int64_t c, int64_t& out, int depth = 0) {
+  if (depth > 16 || v->type.numel() != 1) return false;
+  if (v == counter) { out = c; return true; }
+  if (constantInt(v, out)) return true;
+  Op* d = v->def;
+  if (!d || d->results.size() != 1 || !(isSignedInt(v->type.dt) || v->type.dt == DType::Pred)) return false;
+  std::vector<int64_t> in;
+  for (auto* o : d->operands) {
+    int64_t x;
+    if (!indexAt(o, counter, c, x, depth + 1)) return false;
+    in.push_back(x);
+  }
+  const std::string& n = d->name;
+  if (in.size() == 1 && (n == "reshape" || n == "convert" || n == "broadcast_in_dim")) out = in[0];
+  else if (in.size() == 1 && n == "negate") out = -in[0];
+  else if (in.size() == 2 && n == "add") out = in[0] + in[1];
+  else if (in.size() == 2 && n == "subtract") out = in[0] - in[1];
+  else if (in.size() == 2 && n == "multiply") out = in[0] * in[1];
+  else if (in.size() == 2 && n == "minimum") out = std::min(in[0], in[1]);
+  else if (in.size() == 2 && n == "maximum") out = std::max(in[0], in[1]);
+  else if (in.size() == 3 && n == "clamp") out = std::min(std::max(in[1], in[0]), in[2]);
+  else if (in.size() == 3 && n == "select") out = in[0] ? in[1] : in[2];
+  else if (in.size() == 2 && n == "compare" && isSignedInt(d->operands[0]->type.dt)) {
+    const std::string& dir = d->str("direction");
+    out = dir == "LT" ? in[0] < in[1] : dir == "LE" ? in[0] <= in[1] : dir == "GT" ? in[0] > in[1] : dir == "GE" ? in[0] >= in[1] : dir == "EQ" ? in[0] == in[1] : in[0] != in[1];
+  } else return false;
+  if (v->type.dt != DType::Pred && (out > 2147483647ll || out < -2147483648ll)) return false;   // (no wrap-around to follow)
+  return true;
+}
+
+// start index `index` of a window of one in a dim of `extent`, per iteration
+bool positions(const Recurrence& r, Value* index, int64_t extent, std::vector<int64_t>& out) {
+  const Value* counter = r.loop->regions[1]->args[(size_t)r.counter].get();
+  for (int64_t t = 0; t < r.trip; ++t) {
+    int64_t x;
+    if (!indexAt(index, counter, r.counterInit + t * r.counterStep, x)) return false;
+    out.push_back(std::min(std::max<int64_t>(x, 0), extent - 1));
+  }
+  return true;
+}
+
+struct Accumulated {
+  int carry = -1;
+  Op* op = nullptr;             // dot_general over the rows, or reduce over the rows
+  Value* rows = nullptr;        // the value of the body that is stacked
+  bool rowsFirst = false;       // dot_general: it is the left operand
+  Value* other = nullptr;       // dot_general: the tensor outside whose slices are the other operand
+  Value* index = nullptr;       // dot_general: the body's index of the slice
+  std::vector<int64_t> at;      // and its values
+};
+
+struct Matcher {
+  Op* loop;
+  Region& body;
+  Recurrence r;
+  std::vector<Accumulated> sums;
+
+  explicit Matcher(Op* l) : loop(l), body(*l->regions[1]) {}
+
+  Value* invariant(Value* v) const {
+    if (v->argOf == &body) {
+      const size_t k = (size_t)v->defIndex;
+      return body.terminator()->operands[k] == v ? loop->operands[k] : nullptr;
+    }
+    return regionOf(v) == &body ? nullptr : v;
+  }
+
+  int usesInBody(const Value* v) const {
+    int n = 0;
+    for (auto& o : body.ops) {
+      if (!live.count(o.get())) continue;
+      for (auto* x : o->operands) if (x == v) ++n;
+    }
+    return n;
+  }
+
+  std::unordered_set<const Op*> live;   // ops of the body that its results need
+
+  void mark(Value* v) {
+    if (!v->def || v->def->parent != &body || !live.insert(v->def).second) return;
+    for (auto* o : v->def->operands) mark(o);
+  }
+
+  // acc + (product or sum over the rows)
+  bool accumulated(int k, Value* y) {
+    Op* add = y->def;
+    Value* acc = body.args[(size_t)k].get();
+    if (!add || add->parent != &body || add->name != "add" || y->type.dt != DType::F32 || usesInBody(acc) != 1 || usesInBody(y) != 1) return false;
+    Value* x = add->operands[0] == acc ? add->operands[1] : add->operands[1] == acc ? add->operands[0] : nullptr;
+    if (!x || x == acc || !x->def || x->def->parent != &body || usesInBody(x) != 1) return false;
+    Accumulated a;
+    a.carry = k;
+    a.op = x->def;
+    auto fromBody = [&](Value* v) { return v->type.dt == DType::F32 && v->type.rank() == 2 && regionOf(v) == &body && v->def; };
+    if (a.op->name == "reduce") {
+      const char* kind = simpleReduceKind(*a.op);
+      if (!kind || std::string(kind) != "add" || a.op->ints("dimensions") != std::vector<int64_t>{0}) return false;
+      Op* init = a.op->operands[1]->def;
+      if (!init || init->name != "constant") return false;
+      for (uint8_t byte : init->attrs.at("value").dense->bytes) if (byte) return false;
+      a.rows = a.op->operands[0];
+      if (!fromBody(a.rows)) return false;
+    } else if (a.op->name == "dot_general") {
+      if (!a.op->ints("lhs_batch").empty() || a.op->ints("lhs_contract") != std::vector<int64_t>{0} || a.op->ints("rhs_contract") != std::vector<int64_t>{0}) return false;
+      for (int side = 0; side < 2 && !a.rows; ++side) {
+        Value* v = a.op->operands[(size_t)side];
+        Op* rs = a.op->operands[(size_t)(1 - side)]->def;
+        if (!fromBody(v) || !rs || rs->parent != &body || rs->name != "reshape" || !rs->operands[0]->def) continue;
+        Op* ds = rs->operands[0]->def;
+        if (ds->parent != &body || ds->name != "dynamic_slice") continue;
+        Value* whole = invariant(ds->operands[0]);
+        if (!whole || whole->type.dt != DType::F32 || whole->type.rank() != 3 || rs->result()->type.rank() != 2) continue;
+        const auto& sizes = ds->ints("sizes");
+        if (sizes[0] != 1 || sizes[1] != whole->type.dims[1] || sizes[2] != whole->type.dims[2]) continue;
+        if (rs->result()->type.dims != std::vector<int64_t>(whole->type.dims.begin() + 1, whole->type.dims.end())) continue;
+        if (whole->type.dims[0] != r.trip || !positions(r, ds->operands[1], r.trip, a.at)) { a.at.clear(); continue; }
+        std::vector<int64_t> sorted = a.at;
+        std::sort(sorted.begin(), sorted.end());
+        bool each = true;
+        for (int64_t t = 0; t < r.trip; ++t) if (sorted[(size_t)t] != t) each = false;
+        if (!each) { a.at.clear(); continue; }
+        a.rows = v;
+        a.rowsFirst = side == 0;
+        a.other = whole;
+        a.index = ds->operands[1];
+      }
+      if (!a.rows) return false;
+    } else {
+      return false;
+    }
+    if ((int64_t)a.rows->type.bytes() * r.trip > kStackBytes) return false;
+    sums.push_back(a);
+    return true;
+  }
+
+  bool run() {
+    LoopCounter counter;
+    r.loop = loop;
+    r.trip = staticTripCount(loop, &counter);
+    Op* ret = body.terminator();
+    const int n = (int)loop->operands.size();
+    if (r.trip < kRecurrenceTrips || counter.carry < 0 || !ret || (int)ret->operands.size() != n || (int)body.args.size() != n) return false;
+    r.counter = counter.carry;
+    r.counterInit = counter.init;
+    r.counterStep = counter.step;
+    if (!isSignedInt(body.args[(size_t)r.counter]->type.dt)) return false;
+    for (auto& o : body.ops) if (!o->regions.empty() && o->name != "reduce") return false;
+    live.insert(ret);
+    for (auto* v : ret->operands) mark(v);
+    r.kinds.assign((size_t)n, Recurrence::Passed);
+    for (int k = 0; k < n; ++k) {
+      Value* arg = body.args[(size_t)k].get();
+      Value* y = ret->operands[(size_t)k];
+      if (k == r.counter) { r.kinds[(size_t)k] = Recurrence::Counter; continue; }
+      if (y == arg) continue;
+      Op* d = y->def;
+      if (d && d->parent == &body && d->name == "dynamic_update_slice" && d->operands[0] == arg) {
+        // a window [1, ..., rows, columns] at a position along the leading dim; nothing else reads or yields the stack
+        Value* u = d->operands[1];
+        if (usesInBody(arg) != 1 || usesInBody(y) != 1 || y->type.rank() < 3) return false;
+        Recurrence::Stacked st;
+        st.carry = k;
+        st.value = u;
+        if (u->type.rank() != y->type.rank() || u->type.dims[0] != 1) return false;
+        for (int q = 1; q < y->type.rank(); ++q) if (u->type.dims[(size_t)q] != y->type.dims[(size_t)q] || (q < y->type.rank() - 2 && u->type.dims[(size_t)q] != 1)) return false;
+        if (!recurrenceOffset(r, *d, 2, y->type, u->type.dims, st.base, st.step)) return false;
+        const int64_t window = u->type.numel();
+        st.covers = y->type.dims[0] == r.trip && (st.step == window ? st.base == 0 : st.step == -window && st.base == window * (r.trip - 1));
+        r.kinds[(size_t)k] = Recurrence::Stack;
+        r.stacks.push_back(st);
+        continue;
+      }
+      if (accumulated(k, y)) { r.kinds[(size_t)k] = Recurrence::Accumulator; continue; }
+      if (y->type.dt != DType::F32 || y->type.rank() != 2 || y->type.numel() == 0) return false;
+      if (r.rows == 0) { r.rows = y->type.dims[0]; r.width = y->type.dims[1]; }
+      if (y->type.dims[0] != r.rows || y->type.dims[1] != r.width) return false;
+      r.kinds[(size_t)k] = Recurrence::State;
+    }
+    if (r.rows == 0) return false;
+    // without the accumulations, one product is left
+    live.clear();
+    live.insert(ret);
+    for (int k = 0; k < n; ++k) {
+      if (r.kinds[(size_t)k] != Recurrence::Accumulator) mark(ret->operands[(size_t)k]);
+    }
+    for (auto& a : sums) mark(a.rows);
+    for (auto& o : body.ops) {
+      if (!live.count(o.get()) || (o->name != "dot_general" && o->name != "dot")) continue;
+      if (r.dot || o->name != "dot_general") return false;
+      r.dot = o.get();
+    }
+    if (!r.dot) return false;
+    Value* a = r.dot->operands[0];
+    Value* w = r.dot->operands[1];
+    Value* c = r.dot->result();
+    r.weights = invariant(w);
+    const auto& rc = r.dot->ints("rhs_contract");
+    if (!r.weights || a->type.dt != DType::F32 || w->type.dt != DType::F32 || c->type.dt != DType::F32 || a->type.rank() != 2 || w->type.rank() != 2 || c->type.rank() != 2 ||
+        !r.dot->ints("lhs_batch").empty() || r.dot->ints("lhs_contract") != std::vector<int64_t>{1} || rc.size() != 1)
+      return false;
+    if (a->type.dims[0] != r.rows || a->type.dims[1] % r.width != 0 || c->type.dims[1] % r.width != 0) return false;
+    r.contracted = a->type.dims[1] / r.width;
+    r.pieces = c->type.dims[1] / r.width;
+    r.weightK = rc[0] == 0 ? w->type.dims[1] : 1;
+    r.weightN = rc[0] == 0 ? 1 : w->type.dims[1];
+    const int64_t rb = (r.rows + 15) / 16, cb = (r.width + 15) / 16, units = r.contracted * cb;
+    if (r.pieces > 4 || rb * cb > kRecurrenceBlocks || (units + 3) / 4 > 16 || (units + 3) / 4 * 4 * r.pieces > kRecurrenceWeights) return false;
+    for (auto& st : r.stacks) if (st.value->type.dims.back() % r.width != 0 || st.value->type.dims[(size_t)st.value->type.rank() - 2] != r.rows) return false;
+    for (auto& s : sums) if (s.rows->type.dims[0] != r.rows || s.rows->type.dims[1] % r.width != 0) return false;
+    return true;
+  }
+};
+
+Value* addResult(Op* op, const TensorType& t, int& nextId) {
+  auto v = std::make_unique<Value>();
+  v->id = nextId++;
+  v->type = t;
+  v->def = op;
+  v->defIndex = (int)op->results.size();
+  v->name = "%recurrence" + std::to_string(v->id);
+  op->results.push_back(std::move(v));
+  return op->results.back().get();
+}
+
+Attr intsAttr(const std::vector<int64_t>& v) {
+  Attr a;
+  a.kind = Attr::Ints;
+  a.ints = v;
+  return a;
+}
+
+void replaceUses(Region& region, const Value* from, Value* to) {
+  for (auto& o : region.ops) {
+    for (auto& x : o->operands) if (x == from) x = to;
+    for (auto& sub : o->regions) replaceUses(*sub, from, to);
+  }
+}
+
+int usesIn(const Region& region, const Value* v) {
+  int n = 0;
+  for (auto& o : region.ops) {
+    for (auto* x : o->operands) if (x == v) ++n;
+    for (auto& sub : o->regions) n += usesIn(*sub, v);
+  }
+  return n;
+}
+
+int maxId(const Region& r) {
+  int m = -1;
+  for (auto& a : r.args) m = std::max(m, a->id);
+  for (auto& o : r.ops) {
+    for (auto& v : o->results) m = std::max(m, v->id);
+    for (auto& sub : o->regions) m = std::max(m, maxId(*sub));
+  }
+  return m;
+}
+
+// Replaces the loop at position `pos` of `region`.  Returns the number of ops now in its place, 0 if it is left as it is.
+size_t lower(Region& region, size_t pos, int& nextId) {
+  Op* loop = region.ops[pos].get();
+  Matcher m(loop);
+  if (!m.run()) return 0;
+  Recurrence& r = m.r;
+  // the rows of all iterations that accumulations are taken over: one stack per value, at the positions of the slices they meet
+  struct RowStack { Value* rows; std::vector<int64_t> at; Value* result; };
+  std::vector<RowStack> rowStacks;
+  std::vector<size_t> stackOf;
+  for (auto& a : m.sums) {
+    size_t k = 0;
+    while (k < rowStacks.size() && !(rowStacks[k].rows == a.rows && (a.at.empty() || rowStacks[k].at.empty() || rowStacks[k].at == a.at))) ++k;
+    if (k == rowStacks.size()) rowStacks.push_back({a.rows, a.at, nullptr});
+    else if (rowStacks[k].at.empty()) rowStacks[k].at = a.at;
+    stackOf.push_back(k);
+  }
+  for (auto& rs : rowStacks) {
+    Recurrence::Stacked st;
+    const int64_t window = rs.rows->type.numel();
+    st.value = rs.rows;
+    st.covers = true;
+    if (!rs.at.empty()) {
+      st.base = rs.at[0] * window;
+      st.step = r.trip > 1 ? (rs.at[1] - rs.at[0]) * window : 0;
+      for (int64_t t = 0; t < r.trip; ++t) if (rs.at[(size_t)t] * window != st.base + t * st.step) return 0;
+    } else {
+      st.step = window;
+    }
+    r.stacks.push_back(st);
+  }
+  auto info = std::make_shared<RecurrenceOp>();
+  try {
+    info->code = generateRecurrence(r);
+  } catch (const CompileError&) {
+    return 0;      // something in the loop has no form there: it stays a loop
+  }
+  info->label = "loop of " + std::to_string(r.trip) + " as one kernel around dot_general " + r.dot->operands[0]->type.str() + " x " + r.dot->operands[1]->type.str();
+  auto op = std::make_unique<Op>();
+  op->name = "recurrence";
+  op->parent = &region;
+  op->line = loop->line;
+  op->operands = info->code.leaves;
+  const int n = (int)r.kinds.size();
+  std::vector<std::unique_ptr<Op>> behind;
+  std::vector<std::pair<const Value*, Value*>> replaced;
+  for (int k = 0; k < n; ++k) {
+    Value* was = loop->results[(size_t)k].get();
+    switch (r.kinds[(size_t)k]) {
+      case Recurrence::State:
+        op->operands.push_back(loop->operands[(size_t)k]);
+        replaced.push_back({was, addResult(op.get(), was->type, nextId)});
+        ++info->states;
+        break;
+      case Recurrence::Passed: replaced.push_back({was, loop->operands[(size_t)k]}); break;
+      case Recurrence::Counter: {
+        if (usesIn(region, was) == 0) break;
+        auto c = std::make_unique<Op>();
+        c->name = "constant";
+        c->parent = &region;
+        c->line = loop->line;
+        Attr dv;
+        dv.kind = Attr::Dense;
+        dv.dense = std::make_shared<DenseData>();
+        dv.dense->type = was->type;
+        dv.dense->splat = true;
+        const int64_t last = r.counterInit + r.trip * r.counterStep;
+        dv.dense->bytes.assign(dtypeSize(was->type.dt), 0);
+        memcpy(dv.dense->bytes.data(), &last, dv.dense->bytes.size());   // little endian: the low bytes are the value
+        c->attrs["value"] = dv;
+        replaced.push_back({was, addResult(c.get(), was->type, nextId)});
+        behind.push_back(std::move(c));
+        break;
+      }
+      default: break;
+    }
+  }
+  for (size_t q = 0; q < r.stacks.size(); ++q) {
+    auto& st = r.stacks[q];
+    if (st.carry >= 0) {
+      Value* was = loop->results[(size_t)st.carry].get();
+      info->stackInit.push_back(st.covers ? -1 : (int)op->operands.size());
+      if (!st.covers) op->operands.push_back(loop->operands[(size_t)st.carry]);
+      replaced.push_back({was, addResult(op.get(), was->type, nextId)});
+    } else {
+      TensorType t = st.value->type;
+      t.dims.insert(t.dims.begin(), r.trip);
+      info->stackInit.push_back(-1);
+      rowStacks[q - (r.stacks.size() - rowStacks.size())].result = addResult(op.get(), t, nextId);
+    }
+  }
+  for (size_t j = 0; j < m.sums.size(); ++j) {
+    auto& a = m.sums[j];
+    Value* stack = rowStacks[stackOf[j]].result;
+    Value* was = loop->results[(size_t)a.carry].get();
+    auto whole = std::make_unique<Op>();
+    whole->name = a.op->name;
+    whole->attrs = a.op->attrs;
+    whole->parent = &region;
+    whole->line = a.op->line;
+    if (a.op->name == "reduce") {
+      auto zero = std::make_unique<Op>();
+      Op* init = a.op->operands[1]->def;
+      zero->name = "constant";
+      zero->attrs = init->attrs;
+      zero->parent = &region;
+      zero->line = init->line;
+      whole->operands = {stack, addResult(zero.get(), a.op->operands[1]->type, nextId)};
+      whole->attrs["dimensions"] = intsAttr({0, 1});
+      whole->regions = std::move(a.op->regions);
+      for (auto& sub : whole->regions) sub->parent = whole.get();
+      behind.push_back(std::move(zero));
+    } else {
+      whole->operands = a.rowsFirst ? std::vector<Value*>{stack, a.other} : std::vector<Value*>{a.other, stack};
+      whole->attrs["lhs_contract"] = intsAttr({0, 1});
+      whole->attrs["rhs_contract"] = intsAttr({0, 1});
+    }
+    Value* sum = addResult(whole.get(), was->type, nextId);
+    behind.push_back(std::move(whole));
+    Op* init = loop->operands[(size_t)a.carry]->def;
+    bool zeros = false;      // (an accumulator that starts at zero takes the sum as it is)
+    while (init && init->name == "broadcast_in_dim") init = init->operands[0]->def;
+    if (init && init->name == "constant" && init->attrs.at("value").dense->splat) {
+      zeros = true;
+      for (uint8_t byte : init->attrs.at("value").dense->bytes) if (byte) zeros = false;
+    } else if (init && init->name == "constant" && init->attrs.at("value").dense->type.numel() == 1) {
+      zeros = true;
+      for (uint8_t byte : init->attrs.at("value").dense->bytes) if (byte) zeros = false;
+    }
+    if (!zeros) {
+      auto add = std::make_unique<Op>();
+      add->name = "add";
+      add->operands = {loop->operands[(size_t)a.carry], sum};
+      add->parent = &region;
+      add->line = a.op->line;
+      sum = addResult(add.get(), was->type, nextId);
+      behind.push_back(std::move(add));
+    }
+    replaced.push_back({was, sum});
+  }
+  op->recurrence = info;
+  const size_t placed = 1 + behind.size();
+  std::unique_ptr<Op> old = std::move(region.ops[pos]);
+  region.ops[pos] = std::move(op);
+  region.ops.insert(region.ops.begin() + (long)pos + 1, std::make_move_iterator(behind.begin()), std::make_move_iterator(behind.end()));
+  for (auto& x : replaced) replaceUses(region, x.first, x.second);
+  return placed;
+}
+
+}  // namespace
+
+bool recurrenceOffset(const Recurrence& r, const Op& op, size_t first, const TensorType& type, const std::vector<int64_t>& sizes, int64_t& base, int64_t& step) {
+  const int rank = type.rank();
+  if (op.operands.size() != first + (size_t)rank || (int)sizes.size() != rank) return false;
+  const Value* counter = r.loop->regions[1]->args[(size_t)r.counter].get();
+  std::vector<int64_t> at;
+  for (int64_t t = 0; t < r.trip; ++t) {
+    int64_t off = 0, stride = 1;
+    for (int d = rank - 1; d >= 0; --d) {
+      const int64_t room = type.dims[(size_t)d] - sizes[(size_t)d];
+      if (room > 0) {   // start indices are clamped into range
+        int64_t x;
+        if (!indexAt(op.operands[first + (size_t)d], counter, r.counterInit + t * r.counterStep, x)) return false;
+        off += std::min(std::max<int64_t>(x, 0), room) * stride;
+      }
+      stride *= type.dims[(size_t)d];
+    }
+    at.push_back(off);
+  }
+  base = at[0];
+  step = r.trip > 1 ? at[1] - at[0] : 0;
+  for (int64_t t = 0; t < r.trip; ++t) if (at[(size_t)t] != base + t * step) return false;
+  return true;
+}
+
+bool lowerRecurrences(Module& m) {
+  if (getenv("MI355X_RECURRENCE") && atoi(getenv("MI355X_RECURRENCE")) == 0) return false;
+  Func* f = m.main();
+  if (!f) return false;
+  int nextId = maxId(f->body) + 1;
+  bool any = false;
+  for (size_t k = 0; k < f->body.ops.size(); ++k) {
+    Op* op = f->body.ops[k].get();
+    if (op->name != "while" || op->regions.size() != 2) continue;
+    if (const size_t placed = lower(f->body, k, nextId)) { k += placed - 1; any = true; }
+  }
+  return any;
+}
+
+}  // namespace mi355

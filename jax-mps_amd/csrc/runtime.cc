@@ -226,6 +226,12 @@ DeviceBuffer::~DeviceBuffer() {
 // ------------------------------------------------------------- Executable
 Executable::Executable(std::unique_ptr<CompiledProgram> prog) : prog_(std::move(prog)) {
   Device& dev = Device::get();
+  // Loops as kernels need all their workgroups on the device at once: 128 at most, one per compute unit (two and more fit).
+  if (prog_->loopsAsKernels && dev.computeUnits() >= 128) {
+    auto other = std::move(prog_->loopsAsKernels);
+    prog_ = std::move(other);
+  }
+  prog_->loopsAsKernels.reset();
   const char* t = getenv("MI355X_TIMING");
   timingKinds_ = t ? t : "";
   const char* every = getenv("MI355X_TIMING_EVERY");   // time one execute call in N (sampling keeps the events' own cost small)

@@ -1,0 +1,109 @@
+"""Loops that run as one kernel: batches and widths around the 16 x 16 blocks of a workgroup, one and several blocks each way, a
+single unit of K and units that do not divide by the wavefronts, one to four pieces of the product, a backward loop (several
+pieces of the operand, sums taken out of the loop), stacks written backwards, into a longer tensor and from the product,
+accumulators that do not start at zero, the shortest loop taken, and loops next to it that stay loops (too short, a
+state read at another row)."""
+import numpy as np
+import pytest
+
+from conftest import closeness
+from shlo_oracle import Oracle
+
+pytestmark = pytest.mark.gpu
+
+# name, cell, iterations, rows, width, options
+CASES = [
+    ("one-row", "rnn", 8, 1, 16, ()),
+    ("width-1", "rnn", 9, 5, 1, ()),
+    ("width-15", "rnn", 11, 16, 15, ("reverse",)),
+    ("width-17-rows-17", "rnn", 9, 17, 17, ()),
+    ("blocks", "rnn", 10, 33, 90, ("longer",)),
+    ("most-blocks", "rnn", 8, 128, 256, ()),
+    ("too-many-blocks", "rnn", 8, 130, 256, ()),
+    ("transposed-weights", "rnn", 9, 20, 40, ("transposed",)),
+    ("gates-2", "gated", 12, 20, 33, ()),
+    ("gates-4-wide", "lstm", 9, 18, 130, ()),
+    ("late-stack", "rnn", 10, 20, 24, ("late",)),
+    ("too-short", "rnn", 7, 16, 16, ()),
+    ("other-row", "rnn", 9, 6, 16, ("roll",)),
+    ("backward", "backward", 10, 20, 24, ()),
+    ("backward-pieces", "backward2", 9, 17, 50, ()),
+]
+
+
+def build(cell, trips, rows, width, options):
+    from jax_mps_amd.shlo.builder import Builder
+    b = Builder("recurrence")
+    pieces = {"rnn": 1, "gated": 2, "lstm": 4, "backward": 1, "backward2": 1}[cell]
+    contracted = {"backward2": 3}.get(cell, 1)
+    T = trips + 3 if "longer" in options else trips
+    xs = b.arg((trips, rows, pieces * width), "f32")
+    w = b.arg((width, contracted * width) if "transposed" in options or contracted > 1 else (contracted * width, pieces * width), "f32")
+    bias = b.arg((pieces * width,), "f32")
+    h0 = b.arg((rows, width), "f32")
+    z = lambda: b.constant(0, "i32")   # noqa: E731
+    contract = ([1], [1]) if "transposed" in options or contracted > 1 else ([1], [0])
+    slice_of = lambda t, n: b.reshape(b.dynamic_slice(t, [n, z(), z()], [1] + list(t.shape[1:])), t.shape[1:])   # noqa: E731
+    full = lambda v, shape: b.broadcast_in_dim(b.constant(v, "f32"), shape, [])   # noqa: E731
+    if cell.startswith("backward"):
+        acc0 = b.arg((pieces * width, contracted * width), "f32")
+
+        def body(i, g, c, acc, dbias):
+            t = b.sub(trips - 1, i)
+            x = slice_of(xs, t)
+            dz = [b.mul(g, b.sub(1.0, b.mul(x, x)))] + [b.mul(b.tanh(b.add(g, c)), 0.5 * k) for k in range(1, contracted)]
+            if contracted > 1:
+                total = None
+                for k, d in enumerate(dz):
+                    p = b.pad(d, 0.0, [0, k * width], [0, (contracted - 1 - k) * width])
+                    total = p if total is None else b.add(total, p)
+            else:
+                total = dz[0]
+            prev = b.add(b.dot_general(total, w, contract), b.broadcast_in_dim(bias, (rows, width), [1]))
+            return [b.add(i, 1), prev, b.mul(b.add(c, g), 0.5), b.add(acc, b.dot_general(x, total, ([0], [0]))), b.add(dbias, b.reduce_sum(total, [0]))]
+        out = b.while_loop([z(), h0, full(0.25, (rows, width)), acc0, b.zeros((contracted * width,))], lambda i, *_: b.compare(i, trips, "LT"), body)
+        b.ret(*out)
+        return b.text()
+
+    def body(i, h, c, hs):
+        x = slice_of(xs, i)
+        src = b.concatenate([b.slice(h, [1, 0], [rows, width]), b.slice(h, [0, 0], [1, width])], 0) if "roll" in options else h
+        pre = b.add(b.add(x, b.dot_general(src, w, contract)), b.broadcast_in_dim(bias, (rows, pieces * width), [1]))
+        p = [b.slice(pre, [0, k * width], [rows, (k + 1) * width]) for k in range(pieces)]
+        if cell == "rnn":
+            c2 = b.add(b.mul(c, 0.5), h)
+            h2 = b.tanh(p[0])
+        elif cell == "gated":
+            u = b.logistic(p[0])
+            c2 = b.add(b.mul(u, c), b.mul(b.sub(1.0, u), b.tanh(p[1])))
+            h2 = b.maximum(c2, b.mul(h, 0.1))
+        else:
+            c2 = b.add(b.mul(b.logistic(p[1]), c), b.mul(b.logistic(p[0]), b.tanh(p[2])))
+            h2 = b.mul(b.logistic(p[3]), b.tanh(c2))
+        at = b.sub(trips - 1, i) if "reverse" in options else i
+        hs2 = b.dynamic_update_slice(hs, b.reshape(h2 if "late" in options else h, (1, rows, width)), [at, z(), z()])
+        return [b.add(i, 1), h2, c2, hs2]
+    out = b.while_loop([z(), h0, full(0.25, (rows, width)), full(-1.0, (T, rows, width))], lambda i, *_: b.compare(i, trips, "LT"), body)
+    b.ret(*out)
+    return b.text()
+
+
+@pytest.mark.parametrize("case", CASES, ids=[c[0] for c in CASES])
+def test_recurrence(client, case):
+    from jax_mps_amd import runner
+    name, *spec = case
+    text = build(*spec)
+    print("case", name, flush=True)
+    exe = client.compile_and_load(text)
+    for seed in (1, 2):
+        rng = np.random.default_rng(seed)
+        types = [a.split("tensor<")[1].split(">")[0] for a in text[:text.index("->")].split("%arg")[1:]]
+        shapes = [tuple(int(d) for d in t.split("x")[:-1]) for t in types]
+        scale = 1.0 / np.sqrt(spec[3])      # keeps the chain from growing: errors stay those of single iterations
+        ins = [rng.uniform(-1, 1, s).astype(np.float32) * np.float32(scale if k == 1 else 1) for k, s in enumerate(shapes)]
+        got = [runner.download(o) for o in exe.execute(runner.upload(client, ins, ["f32"] * len(ins)))]
+        want = Oracle(text).run(*ins)
+        assert len(got) == len(want)
+        for k, (g, w) in enumerate(zip(got, want)):
+            ratio = closeness(g, w, 2e-5, 2e-5)
+            assert ratio <= 1.0, f"{name}, output {k}: {ratio:.3f} x the bound"
