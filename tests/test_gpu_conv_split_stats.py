@@ -1,0 +1,45 @@
+"""Column statistics from the fold of a convolution whose K is split: two splits, eight and nine (the fold's two forms) and many,
+one row block of rows and ragged last ones, each number of rows per lane, one column quad, ragged and several column blocks, a
+stem whose loaders are scalar, and columns that are no multiple of four (statistics from a pass of their own).  Bar and inputs
+of test_gpu_resnet_layers: forward form, per-feature sum and sum of squares beside the convolution."""
+import numpy as np
+import pytest
+
+from conftest import closeness
+from shlo_oracle import Oracle
+from test_gpu_resnet_layers import build as build_layer
+
+pytestmark = pytest.mark.gpu
+
+# name, batch, input size, in features, out features, window, stride
+CASES = [
+    ("one-row-block", 1, 3, 64, 64, 3, 1),
+    ("one-column-quad", 2, 9, 64, 4, 3, 1),
+    ("ragged-columns", 3, 11, 48, 100, 3, 1),
+    ("several-column-blocks", 2, 7, 64, 260, 3, 1),
+    ("two-splits", 24, 28, 48, 48, 3, 1),
+    ("rows-2", 16, 32, 64, 64, 3, 1),
+    ("rows-4", 29, 33, 32, 64, 3, 1),
+    ("eight-splits", 16, 16, 128, 128, 3, 1),
+    ("nine-splits", 16, 16, 128, 256, 3, 2),
+    ("many-splits", 16, 4, 512, 512, 3, 1),
+    ("one-window", 16, 8, 256, 512, 1, 2),
+    ("scalar-loaders", 5, 12, 3, 20, 3, 1),
+    ("columns-no-quad", 8, 10, 64, 22, 3, 1),
+]
+
+
+def build(batch, size, cin, cout, k, stride):
+    return build_layer("fwd", size, cin, cout, k, stride, 9400 + batch + cout, batch=batch)
+
+
+@pytest.mark.parametrize("case", CASES, ids=[c[0] for c in CASES])
+def test_split_statistics(client, case):
+    from jax_mps_amd import runner
+    name, *spec = case
+    text, ins, names = build(*spec)
+    print("case", name, spec, flush=True)
+    got = [runner.download(o) for o in client.compile_and_load(text).execute(runner.upload(client, ins, ["f32"] * len(ins)))]
+    for n, g, w in zip(names, got, Oracle(text).run(*ins)):
+        ratio = closeness(g, np.asarray(w), 1e-5, 1e-5)
+        assert ratio <= 1.0, f"{name} {n}: {ratio:.3f} x the bound"
