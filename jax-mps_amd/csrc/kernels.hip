@@ -820,10 +820,10 @@ __global__ void __launch_bounds__(256) scatter_fold_short(const u32* __restrict_
 // cut into column chunks, one workgroup each, and many fetches are in flight: four wavefronts stage a round of
 // updates in LDS (32 independent loads per lane), then the first wavefront applies the staged values of its column
 // in order.  Runs of kLongSegment .. kHugeSegment - 1 updates use chunks of 64 columns and rounds of 128 updates
-// (scatter_fold_long); longer ones (the head of a Zipf distribution: a tenth of all updates go to one row) chunks of
+// (foldLongRuns); longer ones (the head of a Zipf distribution: a tenth of all updates go to one row) chunks of
 // 8 columns and rounds of 1024, a wavefront load covering eight updates, with the fetches of the next round issued
 // before the staged one is folded and the update numbers of round r + 1 fetched during round r - 1
-// (scatter_fold_huge).  A run of length >= L contains a multiple of L, so only those positions get a workgroup, and
+// (foldHugeRuns).  A run of length >= L contains a multiple of L, so only those positions get a workgroup, and
 // the first of them inside the run does the work.
 //
 // Workgroup number = position * chunks + column chunk.  The column chunk is the fast index because workgroups with
@@ -908,20 +908,28 @@ __device__ __forceinline__ void foldLongRun(typename P::S* stage, const u32* __r
 }
 
 constexpr int kHugeCols = 8, kHugePerLane = 32;
+constexpr int kStageElems = 8192;   // 1024 updates x 8 columns, or 128 x 64
+static_assert(4 * (64 / kHugeCols) * kHugePerLane * kHugeCols == kStageElems, "a round of a very long run");
+
+// Can the run around position p, a multiple of L, have L updates or more and no earlier multiple of L?  Then it reaches half of L
+// to one side.  Most workgroups stop here, after loads that do not wait for each other (the search for the run's ends takes
+// three more, one after the other: with it ahead of this answer the idle workgroups took most of the launch).
+template <int L>
+__device__ __forceinline__ bool mayOwnRun(const u32* __restrict__ keys, long long p, long long n, u32 key) {
+  const u32 owner = keys[p >= L ? p - L : 0], below = keys[p >= L / 2 ? p - L / 2 : 0], above = keys[p + L / 2 < n ? p + L / 2 : n - 1];
+  return !(p >= L && owner == key) && ((p >= L / 2 && below == key) || (p + L / 2 < n && above == key));
+}
 
 // Very long runs: chunks of 8 columns and rounds of 1024 updates (see above).
 template <typename P>
-__global__ void __launch_bounds__(256) scatter_fold_huge(const u32* __restrict__ keys, const u32* __restrict__ vals, long long n, long long rowElems,
-                                                          int kind, typename P::S* __restrict__ result, const typename P::S* __restrict__ updates, u32 rows, u32 chunks) {
-  typedef typename P::S S;
-  __shared__ S stage[4 * (64 / kHugeCols) * kHugePerLane * kHugeCols];
+__device__ __forceinline__ void foldHugeRuns(typename P::S* stage, unsigned block, const u32* __restrict__ keys, const u32* __restrict__ vals, long long n,
+                                             long long rowElems, int kind, typename P::S* __restrict__ result, const typename P::S* __restrict__ updates, u32 rows, u32 chunks) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const u32 chunk = blockIdx.x % chunks;                       // workgroup number = position * chunks + column chunk
-  const long long p = (long long)(blockIdx.x / chunks) * kHugeSegment;
+  const u32 chunk = block % chunks;                       // workgroup number = position * chunks + column chunk
+  const long long p = (long long)(block / chunks) * kHugeSegment;
   if (p >= n) return;
   const u32 key = keys[p];
-  if (key >= rows) return;
-  if (p >= kHugeSegment && keys[p - kHugeSegment] == key) return;                    // an earlier workgroup owns this run
+  if (!mayOwnRun<kHugeSegment>(keys, p, n, key) || key >= rows) return;
   const long long head = runHead(keys, p, key, lane);
   if (head + kHugeSegment - 1 >= n || keys[head + kHugeSegment - 1] != key) return;   // shorter run: other kernels
   const long long total = runLast(keys, head + kHugeSegment - 1, n, key, lane) - head + 1;
@@ -930,22 +938,20 @@ __global__ void __launch_bounds__(256) scatter_fold_huge(const u32* __restrict__
 
 // Long runs below kHugeSegment: chunks of 64 columns, rounds of 128 updates whose numbers are staged through LDS.
 template <typename P>
-__device__ __forceinline__ void foldLongRuns(unsigned block, const u32* __restrict__ keys, const u32* __restrict__ vals, long long n, long long rowElems,
+__device__ __forceinline__ void foldLongRuns(typename P::S (*stage)[64], unsigned block, const u32* __restrict__ keys, const u32* __restrict__ vals, long long n, long long rowElems,
                                              int kind, typename P::S* __restrict__ result, const typename P::S* __restrict__ updates, u32 rows, u32 chunks) {
   typedef typename P::S S;
   constexpr int kWaves = 4, kPerLane = 32, kRound = kWaves * kPerLane;   // 128 updates x 64 columns staged per round
   __shared__ u32 sval[256];
-  __shared__ S stage[kRound][64];
   const u32 chunk = block % chunks;                            // workgroup number = position * chunks + column chunk
   const long long p = (long long)(block / chunks) * kLongSegment;
   if (p >= n) return;
   const u32 key = keys[p];
-  if (key >= rows) return;
-  if (p >= kLongSegment && keys[p - kLongSegment] == key) return;                    // an earlier workgroup owns this run
+  if (!mayOwnRun<kLongSegment>(keys, p, n, key) || key >= rows) return;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const long long head = runHead(keys, p, key, lane);
   if (head + kLongSegment - 1 >= n || keys[head + kLongSegment - 1] != key) return;   // short run
-  if (head + kHugeSegment - 1 < n && keys[head + kHugeSegment - 1] == key) return;    // very long run: scatter_fold_huge
+  if (head + kHugeSegment - 1 < n && keys[head + kHugeSegment - 1] == key) return;    // very long run: foldHugeRuns
   const long long col = (long long)chunk * 64 + lane;
   const bool active = col < rowElems;
   const long long colc = active ? col : rowElems - 1;
@@ -985,25 +991,17 @@ __device__ __forceinline__ void foldLongRuns(unsigned block, const u32* __restri
   if (w == 0 && active) result[(long long)key * rowElems + col] = P::store(acc);
 }
 
+// The long and the very long runs in one launch, the very long ones first: both are chains of fetches of a few workgroups with
+// the same LDS, and side by side they take the time of the longer (8192 Zipf-distributed updates of 768 columns: 20 and 12 us
+// apart, 25.5 together).
+// The short runs, of many workgroups without LDS, stay a launch of their own (as the halves of one grid 26 us, apart 23).
 template <typename P>
 __global__ void __launch_bounds__(256) scatter_fold_long(const u32* __restrict__ keys, const u32* __restrict__ vals, long long n, long long rowElems,
-                                                         int kind, typename P::S* __restrict__ result, const typename P::S* __restrict__ updates, u32 rows, u32 chunks) {
-  foldLongRuns<P>(blockIdx.x, keys, vals, n, rowElems, kind, result, updates, rows, chunks);
-}
-
-// Runs below kHugeSegment, short and long, in one launch: workgroups [0, blocksLong) take the long runs, the rest the
-// short ones (run head = rest / chunksShort, 256-column chunk = rest % chunksShort).  The two classes touch different
-// rows and each is a short chain of dependent fetches, so side by side they take the time of one.
-template <typename P>
-__global__ void __launch_bounds__(256) scatter_fold_runs(const u32* __restrict__ keys, const u32* __restrict__ vals, long long n, long long rowElems,
                                                          int kind, typename P::S* __restrict__ result, const typename P::S* __restrict__ updates, u32 rows,
-                                                         u32 chunksLong, u32 blocksLong, u32 chunksShort) {
-  if (blockIdx.x < blocksLong) {
-    foldLongRuns<P>(blockIdx.x, keys, vals, n, rowElems, kind, result, updates, rows, chunksLong);
-    return;
-  }
-  const u32 rest = blockIdx.x - blocksLong;
-  foldShortRuns<P>(rest / chunksShort, rest % chunksShort, keys, vals, n, rowElems, kind, result, updates, rows);
+                                                         u32 chunksHuge, u32 blocksHuge, u32 chunksLong) {
+  __shared__ typename P::S stage[kStageElems];
+  if (blockIdx.x < blocksHuge) foldHugeRuns<P>(stage, blockIdx.x, keys, vals, n, rowElems, kind, result, updates, rows, chunksHuge);
+  else foldLongRuns<P>((typename P::S(*)[64])stage, blockIdx.x - blocksHuge, keys, vals, n, rowElems, kind, result, updates, rows, chunksLong);
 }
 
 // ---- few updates: no sort, one launch ----------------------------------------------------------------------
@@ -1465,7 +1463,7 @@ int mi355_scatter_rows_fill(const mi355_scatter_desc* d, void* result, const voi
   // grids of the fold launches, checked before anything is enqueued
   const long long chunksHuge = (d->rowElems + kHugeCols - 1) / kHugeCols, chunksLong = (d->rowElems + 63) / 64;
   const long long blocksHuge = chunksHuge * ((n + kHugeSegment - 1) / kHugeSegment), blocksLong = chunksLong * ((n + kLongSegment - 1) / kLongSegment);
-  if (blocksHuge > 0x7FFFFFFFll || blocksLong > 0x7FFFFFFFll || n > 0x7FFFFFFFll || (d->rowElems + 255) / 256 > 65535)
+  if (blocksHuge + blocksLong > 0x7FFFFFFFll || n > 0x7FFFFFFFll || (d->rowElems + 255) / 256 > 65535)
     return MI355_SCATTER_GRID_TOO_LARGE;
   const unsigned long long fillBytes = fill ? (unsigned long long)d->operandRows * d->rowElems * elemBytes : 0;
   if (elemBytes == 2) fillBits = (fillBits & 0xFFFFu) | (fillBits << 16);
@@ -1510,19 +1508,10 @@ int mi355_scatter_rows_fill(const mi355_scatter_desc* d, void* result, const voi
     t = vin; vin = vout; vout = t;
   }
   dim3 gridShort((unsigned)n, (unsigned)((d->rowElems + 255) / 256));
-  const long long chunksShort = (d->rowElems + 255) / 256, blocksRuns = blocksLong + n * chunksShort;
-  // (measured on 8192 Zipf-distributed updates of 768 columns: 26 us together against 11.7 + 11.6 us apart, so one launch is
-  // kept for callers that ask for it)
-  static const bool oneLaunch = getenv("MI355X_SCATTER_ONE_FOLD") && getenv("MI355X_SCATTER_ONE_FOLD")[0] == '1';
-  const bool together = oneLaunch && n >= kLongSegment && blocksRuns <= 0x7FFFFFFFll;
+  const long long huge = n >= kHugeSegment ? blocksHuge : 0;
 #define FOLD(P) do { \
-    if (n >= kHugeSegment) scatter_fold_huge<P><<<(unsigned)blocksHuge, 256, 0, st>>>(kin, vin, n, d->rowElems, d->kind, (typename P::S*)result, (const typename P::S*)updates, (u32)d->operandRows, (u32)chunksHuge); \
-    if (together) { \
-      scatter_fold_runs<P><<<(unsigned)blocksRuns, 256, 0, st>>>(kin, vin, n, d->rowElems, d->kind, (typename P::S*)result, (const typename P::S*)updates, (u32)d->operandRows, (u32)chunksLong, (u32)blocksLong, (u32)chunksShort); \
-    } else { \
-      if (n >= kLongSegment) scatter_fold_long<P><<<(unsigned)blocksLong, 256, 0, st>>>(kin, vin, n, d->rowElems, d->kind, (typename P::S*)result, (const typename P::S*)updates, (u32)d->operandRows, (u32)chunksLong); \
-      scatter_fold_short<P><<<gridShort, 256, 0, st>>>(kin, vin, n, d->rowElems, d->kind, (typename P::S*)result, (const typename P::S*)updates, (u32)d->operandRows); \
-    } \
+    if (n >= kLongSegment) scatter_fold_long<P><<<(unsigned)(huge + blocksLong), 256, 0, st>>>(kin, vin, n, d->rowElems, d->kind, (typename P::S*)result, (const typename P::S*)updates, (u32)d->operandRows, (u32)chunksHuge, (u32)huge, (u32)chunksLong); \
+    scatter_fold_short<P><<<gridShort, 256, 0, st>>>(kin, vin, n, d->rowElems, d->kind, (typename P::S*)result, (const typename P::S*)updates, (u32)d->operandRows); \
   } while (0)
   if (d->dtype == 0) FOLD(Plain<float>);
   else if (d->dtype == 2) FOLD(Plain<int>);
