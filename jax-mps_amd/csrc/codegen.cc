@@ -455,6 +455,31 @@ class Emitter {
     std::string ptr = "in" + std::to_string(id);
     IdxDim off = idx.linear ? idx.lin : linearize(idx.dims, leaf->type.dims);
     bool inB = off.inBody || guard_ > 0;
+    const auto parts = splitStored().find(leaf);
+    if (parts != splitStored().end()) {
+      const std::string stride = std::to_string(leaf->type.numel());
+      const bool vec = !inB && off.coef == 1 && V_ > 1 && !off.isConst && off.mult % V_ == 0 && leaf->type.numel() % V_ == 0;
+      std::string sum;
+      for (int p = 0; p < parts->second; ++p) {
+        const std::string at = (vec ? off.base : dimExpr(off)) + " + " + std::to_string(p) + " * " + stride;
+        if (!vec) { sum += (p ? " + " : "") + ptr + "[" + at + "]"; continue; }
+        const std::string key = ptr + "#" + std::to_string(p) + "@" + off.base;
+        auto it = vecLoads_.find(key);
+        if (it == vecLoads_.end()) {
+          it = vecLoads_.emplace(key, fresh("lv")).first;
+          pre("const Vec<float, " + std::to_string(V_) + "> " + it->second + " = *(const Vec<float, " + std::to_string(V_) + ">*)(" + ptr + " + " + at + ");");
+        }
+        sum += (p ? " + " : "") + it->second + ".e[v]";
+      }
+      const std::string t = fresh("ld");
+      if (!vec && !inB && off.coef == 0) {
+        pre("const " + computeT(dt) + " " + t + " = " + roundTo(dt, sum) + ";");
+        return t;
+      }
+      bodyNames_.insert(t);
+      body("const " + computeT(dt) + " " + t + " = " + roundTo(dt, sum) + ";");
+      return t;
+    }
     if (!inB && off.coef == 1 && V_ > 1 && !off.isConst && off.mult % V_ == 0 && leaf->type.numel() % V_ == 0) {
       // one aligned vector load per thread, hoisted out of the lane loop
       std::string key = ptr + "@" + off.base;
@@ -965,7 +990,8 @@ std::string kernelHeader(const std::vector<Value*>& leaves, const std::vector<st
   std::string s = "extern \"C\" __global__ void __launch_bounds__(256) k(";
   bool first = true;
   for (size_t i = 0; i < leaves.size(); ++i) {
-    s += std::string(first ? "" : ", ") + "const " + storageT(leaves[i]->type.dt) + "* __restrict__ in" + std::to_string(i);
+    const bool parts = splitStored().count(leaves[i]) != 0;
+    s += std::string(first ? "" : ", ") + "const " + (parts ? std::string("float") : storageT(leaves[i]->type.dt)) + "* __restrict__ in" + std::to_string(i);
     first = false;
   }
   for (auto& o : outs) {
@@ -984,6 +1010,11 @@ void collectAllValues(Value* root, const LeafPredicate& isLeaf, std::vector<Valu
 }
 
 }  // namespace
+
+std::unordered_map<const Value*, int>& splitStored() {
+  static thread_local std::unordered_map<const Value*, int> m;
+  return m;
+}
 
 bool isFusibleOp(const Op& op) {
   static const char* names[] = {

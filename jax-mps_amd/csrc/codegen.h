@@ -10,6 +10,7 @@
 
 #include <functional>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include <cstdlib>
@@ -25,6 +26,10 @@ inline bool strictBf16() {
   return e && e[0] == '1';
 }
 
+
+// Values in memory as several float32 partial results one after the other, with their number: generated kernels add them in
+// order and round the sum to the value's type where they load it.  Of the program being planned.
+std::unordered_map<const Value*, int>& splitStored();
 
 struct KArg {
   enum Kind { In, Out, Work } kind = In;

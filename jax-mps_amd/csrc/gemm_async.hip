@@ -30,6 +30,7 @@
 // (vmcnt(0)) before the first operand read of each iteration, which serialises load and math.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
@@ -61,6 +62,7 @@ struct AsyncArgs {
   int outBf16;
   int tilesM, tilesN;
   long long total;
+  int split = 1;           // few-tile kernel: K shared out to this many workgroups per tile, float32 partial results [split][batch][M][N]
   int act;                 // 1: y = actA * x * (1 + tanh(actC * (x + actB * x^3))) on the stored value (bf16 results)
   float actA, actB, actC;
 };
@@ -356,7 +358,9 @@ __global__ void __launch_bounds__(kFewWaves * 64) gemm_bf16_few(AsyncArgs g) {
   unsigned id = blockIdx.x;
   const unsigned total = (unsigned)g.total;
   if ((total & 7u) == 0) id = (id & 7u) * (total >> 3) + (id >> 3);   // neighbouring column tiles, which share cache lines of B, on one XCD
-  const unsigned perBatch = (unsigned)g.tilesM * (unsigned)g.tilesN;
+  const unsigned perBatch = (unsigned)g.tilesM * (unsigned)g.tilesN, perSplit = total / (unsigned)g.split;
+  const unsigned part_k = id / perSplit;
+  id -= part_k * perSplit;
   const unsigned bz = id / perBatch, t = id - bz * perBatch;
   const unsigned tn = t / (unsigned)g.tilesM, tm = t - tn * (unsigned)g.tilesM;
   const long long b0 = bz / (unsigned)g.batch1, b1 = bz - (unsigned)b0 * (unsigned)g.batch1;
@@ -385,7 +389,8 @@ __global__ void __launch_bounds__(kFewWaves * 64) gemm_bf16_few(AsyncArgs g) {
       srcB[j] = B + n * g.bLd + (lane >> 4) * 8;
     }
   }
-  const int slabs = (int)(g.K / 32), firstSlab = slabs * wave / NW, mine = slabs * (wave + 1) / NW - firstSlab;
+  const int slabs = (int)(g.K / 32), lowSlab = slabs * (int)part_k / g.split, ownSlabs = slabs * ((int)part_k + 1) / g.split - lowSlab;
+  const int firstSlab = lowSlab + ownSlabs * wave / NW, mine = lowSlab + ownSlabs * (wave + 1) / NW - firstSlab;
   uint4v ra[kDepth][TMB], rb[kDepth][2];
   auto load = [&](auto set, int it) {
     constexpr int S = decltype(set)::value;
@@ -456,7 +461,7 @@ __global__ void __launch_bounds__(kFewWaves * 64) gemm_bf16_few(AsyncArgs g) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) part[wave * kTile + (i * 16 + (lane >> 4) * 4 + e) * 32 + 16 * j + (lane & 15)] = acc[i][j][e];
   __syncthreads();
-  const long long cBase = (long long)bz * g.M * g.N;
+  const long long cBase = ((long long)part_k * (perSplit / perBatch) + bz) * g.M * g.N;
 #pragma unroll
   for (int u = tid; u < kTile / 2; u += NW * 64) {
     const long long row = m0 + (u >> 4), col = n0 + (u & 15) * 2;
@@ -597,6 +602,7 @@ extern "C" size_t mi355_gemm_bf16_async_workspace_bytes(const mi355_gemm_desc* d
 
 // The kernel for few output tiles of 16-bit products whose lhs rows are k-contiguous and whose rhs is contiguous either way, all
 // 16-byte loads, K in whole slabs (0 = launched, -1 = not one of its shapes).
+// With d->split > 1 K is shared out to that many workgroups per tile, whose float32 partial results the reader adds.
 static int launchFew(const mi355_gemm_desc* d, const void* a, const void* b, void* c, const void* bias, hipStream_t st) {
   if (d->in_dtype != 1 || (d->out_dtype != 0 && d->out_dtype != 1) || (d->act && d->out_dtype != 1)) return -1;
   const long long nb = d->batch0 * d->batch1;
@@ -618,8 +624,10 @@ static int launchFew(const mi355_gemm_desc* d, const void* a, const void* b, voi
   const int most = d->K >= 768 ? 4 : rowsOfK ? 3 : 2;
   int tmb = 1;
   while (tmb <= most && (blocks + tmb - 1) / tmb * tilesN * nb > kUnits) ++tmb;
-  if (tmb > most) return -1;
+  if (d->split > 1) tmb = (int)blocks;   // (four at most: mi355_gemm_few_split) all rows in one workgroup, so that the rhs is read once
+  else if (tmb > most) return -1;
   AsyncArgs g;
+  g.split = d->split > 1 ? d->split : 1;
   g.a = (const u16*)a; g.b = (const u16*)b; g.c = c; g.bias = bias;
   g.M = d->M; g.N = d->N; g.K = d->K;
   g.aB0 = d->aB0; g.aB1 = d->aB1; g.aLd = d->aRow;
@@ -629,13 +637,27 @@ static int launchFew(const mi355_gemm_desc* d, const void* a, const void* b, voi
   g.act = d->act; g.actA = d->act_a; g.actB = d->act_b; g.actC = d->act_c;
   g.tilesM = (int)((blocks + tmb - 1) / tmb);
   g.tilesN = (int)tilesN;
-  g.total = (long long)g.tilesM * g.tilesN * nb;
+  g.total = (long long)g.tilesM * g.tilesN * nb * g.split;
+  if (g.split > 1) g.outBf16 = 0;
   const dim3 grid((unsigned)g.total);
 #define FEW(TMB) do { \
   if (rowsOfK) gemm_bf16_few<TMB, true><<<grid, kFewWaves * 64, 0, st>>>(g); else gemm_bf16_few<TMB, false><<<grid, kFewWaves * 64, 0, st>>>(g); } while (0)
   if (tmb == 1) FEW(1); else if (tmb == 2) FEW(2); else if (tmb == 3) FEW(3); else FEW(4);
 #undef FEW
   return hipGetLastError() == hipSuccess ? 0 : 3;
+}
+
+// Into how many parts K of a 16-bit product of at most 64 rows is split when its reader can add the parts (0: it is not).  A compute
+// unit takes in about 15 bytes a cycle: unsplit, 24 column tiles of a 768-wide result and K = 3072 leave 72 workgroups 294 KB
+// each; in eight parts with all rows together 192 workgroups take 61 KB each: 8.6 -> 5.4 us,
+// and 5.8 -> 4.8 for K = 768 in four; the normalisation that adds the parts takes 3.6 us as it did.  Parts of at least six slabs.
+extern "C" int mi355_gemm_few_split(const mi355_gemm_desc* d) {
+  const long long nb = d->batch0 * d->batch1, blocks = (d->M + 15) / 16, tilesN = (d->N + 31) / 32, slabs = d->K / 32;
+  if (d->in_dtype != 1 || d->out_dtype != 1 || d->act || nb != 1 || d->M <= 0 || d->N <= 0 || blocks > 4 || d->K % 32 != 0) return 0;
+  const bool rowsOfK = d->bCol == 1 && d->bRow % 8 == 0 && d->N % 8 == 0 && d->bRow >= d->N, kContiguous = d->bRow == 1 && d->bCol % 8 == 0;
+  if (d->aCol != 1 || d->aRow % 8 || (!rowsOfK && !kContiguous)) return 0;
+  const long long parts = std::min<long long>(std::min<long long>(8, 256 / tilesN), slabs / 6);
+  return parts >= 2 ? (int)parts : 0;
 }
 
 // 0 = launched, -1 = layout does not qualify, other = launch error.
@@ -645,6 +667,7 @@ extern "C" int mi355_gemm_bf16_async(const mi355_gemm_desc* d, const void* a, co
   const int wideMode = getenv("MI355X_GEMM_WIDE") ? atoi(getenv("MI355X_GEMM_WIDE")) : 1;   // both read at every call: tests switch them
   const bool fewOn = !getenv("MI355X_GEMM_FEW") || atoi(getenv("MI355X_GEMM_FEW")) != 0;
   const bool wideForced = wideMode == 2 && d->M >= 256 && d->N >= 256;
+  if (d->split > 1) return launchFew(d, a, b, c, nullptr, (hipStream_t)s);
   if (!force && fewOn && !wideForced)                      // (a forced tiling is one of the ring kernel's)
     if (const int few = launchFew(d, a, b, c, bias, (hipStream_t)s); few >= 0) return few;
   OperandPlan pa, pb;

@@ -73,7 +73,11 @@ typedef struct {
   // act 2 (small fp32 products only, mi355_gemm_is_small): y = maximum(x, 0)
   int act;
   float act_a, act_b, act_c;
+  // > 1 (mi355_gemm_few_split): C holds that many float32 partial results one after the other, and whoever reads it adds
+  // them in order and rounds the sum to out_dtype; no bias, no act
+  int split;
 } mi355_gemm_desc;
+int mi355_gemm_few_split(const mi355_gemm_desc* d);
 // `workspace` (may be NULL) holds k-contiguous copies of bf16 operands; see mi355_gemm_workspace_bytes.
 // `bias` (may be NULL): N values of the output type added to every row of C after the product has been rounded to
 // the output type, i.e. exactly dot_general followed by add(broadcast(bias)).

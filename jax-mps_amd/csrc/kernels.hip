@@ -1367,6 +1367,7 @@ int mi355_gemm(const mi355_gemm_desc* d, const void* a, const void* b, void* c, 
   if (d->in_dtype == 1) {
     int r = mi355_gemm_bf16_async(d, a, b, c, bias, workspace, workspace_bytes, s);
     if (r >= 0) return r;
+    if (d->split > 1) return 2;   // (operands are not aligned as planned: no other kernel writes partial results)
     r = mi355_gemm_bf16_tiled(d, a, b, c, s);
     if (r >= 0) return r ? r : addBias(d, c, bias, s);
   }

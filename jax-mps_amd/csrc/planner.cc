@@ -66,6 +66,7 @@ class Planner {
     Func* main = P.module->main();
     Region& body = main->body;
     ivArgs().clear();
+    splitStored().clear();
     rebuildUses(body);
     for (auto& a : body.args) {
       P.paramTypes.push_back(a->type);
@@ -1842,6 +1843,41 @@ class Planner {
     emitDotStep(op, plan, d, nullptr, nullptr);
   }
 
+  // A bf16 product of few rows that only a residual sum reads, after its bias (the projection ahead of a normalisation): K is
+  // shared out to several workgroups per tile, and the generated kernel that reads the product adds the parts and the bias.
+  bool emitSplitDot(Op* op, Plan& plan, const DotPlan& dp) {
+    Value* c = op->result();
+    const char* few = getenv("MI355X_GEMM_FEW");
+    if ((few && atoi(few) == 0) || getenv("MI355X_GEMM_TILE") || loopDepth_ != 0 || dp.rhsFreeDims != 1) return false;
+    if (!dp.va.iterOffsets.empty() || !dp.vb.iterOffsets.empty() || dp.va.offset % 8 || dp.vb.offset % 8) return false;
+    mi355_gemm_desc abi = toAbi(dp.g);
+    const int parts = c->type.numel() > 0 ? mi355_gemm_few_split(&abi) : 0;
+    if (parts < 2) return false;
+    Op* biasAdd = biasAddOf(c);
+    if (!biasAdd || c->users.size() != 1 || needMat_[biasAdd->result()]) return false;
+    Value* other = biasAdd->operands[0] == c ? biasAdd->operands[1] : biasAdd->operands[0];
+    if (!hasStorage(other->def->operands[0]) || needMat_[other]) return false;
+    Value* y = biasAdd->result();
+    while (y->users.size() == 1 && (y->users[0]->name == "reshape" || y->users[0]->name == "convert") && y->users[0]->parent == op->parent && !needMat_[y->users[0]->result()])
+      y = y->users[0]->result();
+    if (y->users.size() != 1 || y->users[0]->name != "add" || y->users[0]->parent != op->parent || y->users[0]->operands[0] == y->users[0]->operands[1]) return false;
+    const int sid = newStorage((size_t)c->type.numel() * 4 * (size_t)parts);
+    bind(c, sid);
+    splitStored()[c] = parts;
+    const int t = ++time_;
+    Step s;
+    s.kind = Step::Gemm;
+    s.time = t;
+    s.label = "dot_general " + op->operands[0]->type.str() + " x " + op->operands[1]->type.str() + " in " + std::to_string(parts) + " parts";
+    s.gemm = dp.g;
+    s.gemm.split = parts;
+    s.args = {ref(storageOf(dp.va.root), t), ref(storageOf(dp.vb.root), t), ref(sid, t)};
+    s.args[0].offset = dp.va.offset * 2;
+    s.args[1].offset = dp.vb.offset * 2;
+    plan.steps.push_back(std::move(s));
+    return true;
+  }
+
   void emitDotStep(Op* op, Plan& plan, const DotPlan& dp, Op* second, const DotPlan* dp2) {
     Value* a = op->operands[0];
     Value* b = op->operands[1];
@@ -1856,6 +1892,7 @@ class Planner {
       sumAdd = c->users[0];
       produced = sumAdd->result();
     }
+    if (!second && emitSplitDot(op, plan, dp)) return;
     // product -> add(broadcast(bias over the last dim)) with no other reader of the product: the kernels add the
     // bias while they store the result (the reference fuses the same pair into one addmm, passes/fuse_bias_add.cc:120-171)
     Value* biasV = nullptr;
@@ -2987,6 +3024,7 @@ mi355_gemm_desc toAbi(const GemmDesc& g) {
   d.in_dtype = abiDtypeCode(g.inType);
   d.out_dtype = abiDtypeCode(g.outType);
   d.act = g.act; d.act_a = g.actA; d.act_b = g.actB; d.act_c = g.actC;
+  d.split = g.split;
   return d;
 }
 

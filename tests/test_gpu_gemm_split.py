@@ -1,0 +1,89 @@
+"""bf16 products of at most 64 rows whose K is shared out to several workgroups, the reader adding the float32 parts: two parts
+and the most, one to four row blocks, ragged rows and columns (vector and scalar loads of the parts), both layouts of the
+right-hand side, read by a normalised residual sum and by one that is stored, and the shapes and readers next to it that stay
+whole (65 rows, K of eleven slabs, no residual, a second reader)."""
+import numpy as np
+import pytest
+
+from shlo_oracle import round_bf16
+
+pytestmark = pytest.mark.gpu
+
+# name, rows, K, N, k-contiguous rhs, reader
+CASES = [
+    ("one-row", 1, 384, 64, False, "norm"),
+    ("rows-17", 17, 768, 768, False, "norm"),
+    ("rows-37-long-k", 37, 3072, 768, False, "norm"),
+    ("rows-48-nt", 48, 1536, 256, True, "norm"),
+    ("rows-64-most-columns", 64, 416, 2048, False, "norm"),
+    ("stored", 33, 800, 72, False, "sum"),
+    ("stored-odd-columns-nt", 20, 544, 45, True, "sum"),
+    ("rank-3", 37, 768, 96, False, "rank-3"),
+    ("rows-65", 65, 768, 64, False, "norm"),
+    ("short-k", 16, 352, 64, False, "norm"),
+    ("no-residual", 16, 768, 64, False, "bias"),
+    ("two-readers", 16, 768, 64, False, "twice"),
+]
+
+
+def build(rows, k, n, nt, reader):
+    from jax_mps_amd.shlo.builder import Builder, layer_norm
+    b = Builder("gemm_split")
+    lead = (1, rows) if reader == "rank-3" else (rows,)
+    x = b.arg(lead + (k,), "bf16")
+    w = b.arg((n, k) if nt else (k, n), "bf16")
+    bias, res = b.arg((n,), "bf16"), b.arg(lead + (n,), "bf16")
+    y = b.dot_general(x, w, ([len(lead)], [1 if nt else 0]))
+    y = b.add(y, b.broadcast_in_dim(bias, lead + (n,), [len(lead)]))
+    if reader == "bias":
+        b.ret(y)
+    elif reader == "sum":
+        b.ret(b.add(res, y))
+    elif reader == "twice":
+        b.ret(b.add(res, y), b.mul(y, y))
+    else:
+        scale, shift = b.arg((n,), "bf16"), b.arg((n,), "bf16")
+        b.ret(layer_norm(b, b.add(res, y), scale, shift, 1e-12))
+    return b.text()
+
+
+def exact_and_bound(spec, x, w, bias, res=None, scale=None, shift=None):
+    """The results in float64, and what the program's own bf16 roundings (half of 2^-7 relative each) may move them by: the product, its
+    sum with the bias and that with the residual round once each; the normalised value moves with its row's own error, the mean's
+    and the deviation's, and rounds once itself, times scale once, plus shift once.  Float32 sums add below 1e-4; second-order
+    terms are within 2 %."""
+    u, reader = 2.0 ** -8, spec[4]
+    x, w, bias = x.astype(np.float64), w.astype(np.float64), bias.astype(np.float64)
+    p = x @ (w.T if spec[3] else w)
+    pb = p + bias
+    if reader == "bias":
+        return [(pb, u * (abs(p) + abs(pb)) * 1.02 + 1e-4)]
+    y = pb + res
+    e = u * (abs(p) + abs(pb) + abs(y))
+    if reader == "sum":
+        return [(y, e * 1.02 + 1e-4)]
+    if reader == "twice":
+        return [(y, e * 1.02 + 1e-4), (pb * pb, u * (2 * abs(pb) * (abs(p) + abs(pb)) + pb * pb) * 1.02 + 1e-4)]
+    std = np.sqrt(y.var(-1, keepdims=True) + 1e-12)
+    h = (y - y.mean(-1, keepdims=True)) / std
+    dh = (e + e.mean(-1, keepdims=True)) / std + abs(h) * np.sqrt((e * e).mean(-1, keepdims=True)) / std + u * abs(h)
+    out = h * scale + shift
+    return [(out, (abs(scale) * dh + u * abs(h * scale) + u * abs(out)) * 1.02 + 1e-4)]
+
+
+@pytest.mark.parametrize("case", CASES, ids=[c[0] for c in CASES])
+def test_split(client, case):
+    from jax_mps_amd import runner
+    name, *spec = case
+    text = build(*spec)
+    rng = np.random.default_rng(len(name))
+    shapes = [tuple(int(d) for d in a.split("tensor<")[1].split(">")[0].split("x")[:-1]) for a in text[:text.index("->")].split("%arg")[1:]]
+    ins = [round_bf16(rng.standard_normal(s).astype(np.float32) / (np.float32(spec[1]) ** 0.25 if i < 2 else 1)) for i, s in enumerate(shapes)]
+    want = exact_and_bound(spec, *ins)
+    print("case", name, flush=True)
+    exe = client.compile_and_load(text)
+    for _ in range(2):
+        got = [runner.download(o) for o in exe.execute(runner.upload(client, ins, ["bf16"] * len(ins)))]
+        assert len(got) == len(want)
+        for g, (w, bound) in zip(got, want):
+            assert np.all(np.abs(np.asarray(g, np.float64) - w) <= bound), (name, float(np.max(np.abs(g - w) / bound)))
