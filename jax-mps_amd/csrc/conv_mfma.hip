@@ -1186,7 +1186,7 @@ static int launchPart(const ConvPart& part, const void* lhs, const void* rhs, vo
   if (c.bm == 128 && c.bn == 128) launchIgemm<128, 128>(c, p, grid, st);
   else if (c.bm == 128) launchIgemm<128, 64>(c, p, grid, st);
   else launchIgemm<64, 64>(c, p, grid, st);
-  if (c.splitK > 1) {
+  if (c.splitK > 1 && out) {   // (without `out` the partial results stay in the workspace: mi355_conv_parts)
     long long total = M * d->O;
     if (statSum) {
       if (bias || part.outOffset || p.N % 4 != 0 || (((uintptr_t)workspace | (uintptr_t)dst) & 15) != 0) return 5;   // (mi355_conv_stats_rows promised otherwise)
@@ -1294,6 +1294,24 @@ int mi355_conv_stats(const mi355_conv_desc* d, const void* lhs, const void* rhs,
 int mi355_conv_bias(const mi355_conv_desc* d, const void* lhs, const void* rhs, void* out, const void* bias, void* workspace,
                     size_t workspace_bytes, mi355_stream_t s) {
   return convolve(d, lhs, rhs, out, workspace, workspace_bytes, nullptr, nullptr, (const float*)bias, s);
+}
+
+// Into how many parts K is split, when the parts can be left in memory as [part][row][feature] for the reader to add in the
+// order of conv_fold_few (0: they cannot).  The fold of 1024 rows of 768 features in five parts took 5.2 us between the
+// product and the normalisation that reads it; adding them there takes the normalisation from 5.1 to 5.3 us (six layers of a
+// float32 encoder 1214 -> 1170 us).  Up to 1.4 million results are split, so reading the parts twice costs what the fold did.
+int mi355_conv_split_parts(const mi355_conv_desc* d) {
+  mi355_conv_desc d2;
+  if (d->O % 4 != 0 || repackedFilter(d, &d2)) return 0;
+  const ConvChoice c = choose(d);
+  if (!c.fast || c.bFast || c.splitK < 2 || c.splitK > 8) return 0;
+  const auto parts = partsOf(d);
+  return parts.size() == 1 && parts[0].outOffset == 0 ? c.splitK : 0;
+}
+
+int mi355_conv_parts(const mi355_conv_desc* d, const void* lhs, const void* rhs, void* results, size_t bytes, mi355_stream_t s) {
+  if (mi355_conv_split_parts(d) == 0) return 5;
+  return launchPart(partsOf(d)[0], lhs, rhs, nullptr, results, bytes, (hipStream_t)s);
 }
 
 }  // extern "C"

@@ -73,10 +73,11 @@ typedef struct {
   // act 2 (small fp32 products only, mi355_gemm_is_small): y = maximum(x, 0)
   int act;
   float act_a, act_b, act_c;
-  // > 1 (mi355_gemm_few_split): C holds that many float32 partial results one after the other, and whoever reads it adds
+  // > 1 (mi355_gemm_split_parts): C holds that many float32 partial results one after the other, and whoever reads it adds
   // them in order and rounds the sum to out_dtype; no bias, no act
   int split;
 } mi355_gemm_desc;
+int mi355_gemm_split_parts(const mi355_gemm_desc* d);
 int mi355_gemm_few_split(const mi355_gemm_desc* d);
 // `workspace` (may be NULL) holds k-contiguous copies of bf16 operands; see mi355_gemm_workspace_bytes.
 // `bias` (may be NULL): N values of the output type added to every row of C after the product has been rounded to
@@ -130,6 +131,9 @@ size_t mi355_conv_workspace_bytes(const mi355_conv_desc* d);
 int mi355_conv_implicit(const mi355_conv_desc* d);
 // The convolution with a value per output feature added to the result (the same sum a later pass over it would make);
 // -1, with nothing launched, where only the direct kernel takes the convolution.  bias may be NULL.
+// K split into that many parts (0: not so), left as [part][row][feature] in `results` for the reader to add in order
+int mi355_conv_split_parts(const mi355_conv_desc* d);
+int mi355_conv_parts(const mi355_conv_desc* d, const void* lhs, const void* rhs, void* results, size_t bytes, mi355_stream_t s);
 int mi355_conv_bias(const mi355_conv_desc* d, const void* lhs, const void* rhs, void* out, const void* bias, void* workspace,
                     size_t workspace_bytes, mi355_stream_t s);
 // Column statistics next to the output: mi355_conv_stats_rows(d) > 0 says the convolution can deliver, for each of that

@@ -1256,6 +1256,14 @@ size_t mi355_gemm_workspace_bytes(const mi355_gemm_desc* d) {
   return 0;
 }
 
+// Into how many parts K is split when the reader can add them (0: it is not, or the kernel adds them itself).  A float32
+// product runs split over K either way; left to the reader its fold is not launched.
+int mi355_gemm_split_parts(const mi355_gemm_desc* d) {
+  if (d->in_dtype == 1) return mi355_gemm_few_split(d);
+  mi355_conv_desc cd;
+  return d->act || smallGemmTile(d) || !gemmAsPointwiseConv(d, &cd) ? 0 : mi355_conv_split_parts(&cd);
+}
+
 static SmallPair smallPair(const mi355_gemm_desc* d, const void* a, const void* b) {
   SmallPair p;
   p.a = (const float*)a; p.b = (const float*)b;
@@ -1376,10 +1384,12 @@ int mi355_gemm(const mi355_gemm_desc* d, const void* a, const void* b, void* c, 
   mi355_conv_desc cd;
   // strided views may start anywhere; the implicit-GEMM loaders issue 16-byte loads
   if (gemmAsPointwiseConv(d, &cd) && (((uintptr_t)a | (uintptr_t)b) & 15) == 0) {
+    if (d->split > 1) return mi355_conv_parts(&cd, a, b, c, (size_t)d->split * (size_t)d->M * (size_t)d->N * sizeof(float), s);
     // the bias rides in the accumulators (or in the fold of a split K): the pass that added it took 4.5 to 7 us per layer
     // of 1024 rows, a tenth of the products' time
     return mi355_conv_bias(&cd, a, b, c, bias, workspace, workspace_bytes, s);
   }
+  if (d->split > 1) return 2;   // (operands are not aligned as planned: no other kernel writes partial results)
   if (nb > 65535) return 1;   // grid.z limit; callers fold larger batches
   // output tiles along x, columns fastest: y ends at 65535, which four million rows reach
   const long long tiles = ((d->N + 63) / 64) * ((d->M + 63) / 64);

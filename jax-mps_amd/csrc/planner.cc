@@ -1843,15 +1843,15 @@ class Planner {
     emitDotStep(op, plan, d, nullptr, nullptr);
   }
 
-  // A bf16 product of few rows that only a residual sum reads, after its bias (the projection ahead of a normalisation): K is
-  // shared out to several workgroups per tile, and the generated kernel that reads the product adds the parts and the bias.
+  // A bf16 product of few rows, or a float32 one whose K is split anyway, that only a residual sum reads, after its bias (the
+  // projection ahead of a normalisation): the generated kernel that reads the product adds the parts and the bias.
   bool emitSplitDot(Op* op, Plan& plan, const DotPlan& dp) {
     Value* c = op->result();
     const char* few = getenv("MI355X_GEMM_FEW");
     if ((few && atoi(few) == 0) || getenv("MI355X_GEMM_TILE") || loopDepth_ != 0 || dp.rhsFreeDims != 1) return false;
     if (!dp.va.iterOffsets.empty() || !dp.vb.iterOffsets.empty() || dp.va.offset % 8 || dp.vb.offset % 8) return false;
     mi355_gemm_desc abi = toAbi(dp.g);
-    const int parts = c->type.numel() > 0 ? mi355_gemm_few_split(&abi) : 0;
+    const int parts = c->type.numel() > 0 ? mi355_gemm_split_parts(&abi) : 0;
     if (parts < 2) return false;
     Op* biasAdd = biasAddOf(c);
     if (!biasAdd || c->users.size() != 1 || needMat_[biasAdd->result()]) return false;
@@ -1872,8 +1872,8 @@ class Planner {
     s.gemm = dp.g;
     s.gemm.split = parts;
     s.args = {ref(storageOf(dp.va.root), t), ref(storageOf(dp.vb.root), t), ref(sid, t)};
-    s.args[0].offset = dp.va.offset * 2;
-    s.args[1].offset = dp.vb.offset * 2;
+    s.args[0].offset = dp.va.offset * (int64_t)dtypeSize(dp.g.inType);
+    s.args[1].offset = dp.vb.offset * (int64_t)dtypeSize(dp.g.inType);
     plan.steps.push_back(std::move(s));
     return true;
   }

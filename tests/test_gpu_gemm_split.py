@@ -1,7 +1,8 @@
-"""bf16 products of at most 64 rows whose K is shared out to several workgroups, the reader adding the float32 parts: two parts
+"""Products whose K is shared out to several workgroups, the reader adding the float32 parts.  bf16 of at most 64 rows: two parts
 and the most, one to four row blocks, ragged rows and columns (vector and scalar loads of the parts), both layouts of the
 right-hand side, read by a normalised residual sum and by one that is stored, and the shapes and readers next to it that stay
-whole (65 rows, K of eleven slabs, no residual, a second reader)."""
+whole (65 rows, K of eleven slabs, no residual, a second reader).  float32: two parts and eight, a ragged K, a right-hand side
+contiguous along K, and what keeps its fold (nine parts, columns not a multiple of four, no residual, a second reader)."""
 import numpy as np
 import pytest
 
@@ -9,30 +10,40 @@ from shlo_oracle import round_bf16
 
 pytestmark = pytest.mark.gpu
 
-# name, rows, K, N, k-contiguous rhs, reader
+# name, rows, K, N, k-contiguous rhs, reader, float32
 CASES = [
-    ("one-row", 1, 384, 64, False, "norm"),
-    ("rows-17", 17, 768, 768, False, "norm"),
-    ("rows-37-long-k", 37, 3072, 768, False, "norm"),
-    ("rows-48-nt", 48, 1536, 256, True, "norm"),
-    ("rows-64-most-columns", 64, 416, 2048, False, "norm"),
-    ("stored", 33, 800, 72, False, "sum"),
-    ("stored-odd-columns-nt", 20, 544, 45, True, "sum"),
-    ("rank-3", 37, 768, 96, False, "rank-3"),
-    ("rows-65", 65, 768, 64, False, "norm"),
-    ("short-k", 16, 352, 64, False, "norm"),
-    ("no-residual", 16, 768, 64, False, "bias"),
-    ("two-readers", 16, 768, 64, False, "twice"),
+    ("one-row", 1, 384, 64, False, "norm", False),
+    ("rows-17", 17, 768, 768, False, "norm", False),
+    ("rows-37-long-k", 37, 3072, 768, False, "norm", False),
+    ("rows-48-nt", 48, 1536, 256, True, "norm", False),
+    ("rows-64-most-columns", 64, 416, 2048, False, "norm", False),
+    ("stored", 33, 800, 72, False, "sum", False),
+    ("stored-odd-columns-nt", 20, 544, 45, True, "sum", False),
+    ("rank-3", 37, 768, 96, False, "rank-3", False),
+    ("rows-65", 65, 768, 64, False, "norm", False),
+    ("short-k", 16, 352, 64, False, "norm", False),
+    ("no-residual", 16, 768, 64, False, "bias", False),
+    ("two-readers", 16, 768, 64, False, "twice", False),
+    ("f32-two-parts", 1000, 400, 516, False, "norm", True),
+    ("f32-eight-parts", 600, 1600, 644, False, "norm", True),
+    ("f32-ragged-k", 520, 804, 520, False, "rank-3", True),
+    ("f32-k-contiguous", 1024, 768, 768, True, "norm", True),
+    ("f32-stored", 1027, 768, 768, False, "sum", True),
+    ("f32-nine-parts", 600, 1744, 644, False, "norm", True),
+    ("f32-columns", 600, 1600, 646, False, "norm", True),
+    ("f32-no-residual", 1000, 400, 516, False, "bias", True),
+    ("f32-two-readers", 1000, 400, 516, False, "twice", True),
 ]
 
 
-def build(rows, k, n, nt, reader):
+def build(rows, k, n, nt, reader, f32):
     from jax_mps_amd.shlo.builder import Builder, layer_norm
     b = Builder("gemm_split")
+    t = "f32" if f32 else "bf16"
     lead = (1, rows) if reader == "rank-3" else (rows,)
-    x = b.arg(lead + (k,), "bf16")
-    w = b.arg((n, k) if nt else (k, n), "bf16")
-    bias, res = b.arg((n,), "bf16"), b.arg(lead + (n,), "bf16")
+    x = b.arg(lead + (k,), t)
+    w = b.arg((n, k) if nt else (k, n), t)
+    bias, res = b.arg((n,), t), b.arg(lead + (n,), t)
     y = b.dot_general(x, w, ([len(lead)], [1 if nt else 0]))
     y = b.add(y, b.broadcast_in_dim(bias, lead + (n,), [len(lead)]))
     if reader == "bias":
@@ -42,28 +53,31 @@ def build(rows, k, n, nt, reader):
     elif reader == "twice":
         b.ret(b.add(res, y), b.mul(y, y))
     else:
-        scale, shift = b.arg((n,), "bf16"), b.arg((n,), "bf16")
+        scale, shift = b.arg((n,), t), b.arg((n,), t)
         b.ret(layer_norm(b, b.add(res, y), scale, shift, 1e-12))
     return b.text()
 
 
 def exact_and_bound(spec, x, w, bias, res=None, scale=None, shift=None):
-    """The results in float64, and what the program's own bf16 roundings (half of 2^-7 relative each) may move them by: the product, its
+    """The results in float64, and what the program's own bf16 roundings (2^-8 relative each) may move them by: the product, its
     sum with the bias and that with the residual round once each; the normalised value moves with its row's own error, the mean's
-    and the deviation's, and rounds once itself, times scale once, plus shift once.  Float32 sums add below 1e-4; second-order
+    and the deviation's, and rounds once itself, times scale once, plus shift once.  In float32 the same steps
+    round by 2^-24 and the product's sum by up to K times that; what else is summed in float32 adds below 1e-4; second-order
     terms are within 2 %."""
-    u, reader = 2.0 ** -8, spec[4]
+    u, reader = 2.0 ** -24 if spec[5] else 2.0 ** -8, spec[4]
     x, w, bias = x.astype(np.float64), w.astype(np.float64), bias.astype(np.float64)
-    p = x @ (w.T if spec[3] else w)
+    w = w.T if spec[3] else w
+    p = x @ w
+    sums = spec[1] * 2.0 ** -24 * (abs(x) @ abs(w))
     pb = p + bias
     if reader == "bias":
-        return [(pb, u * (abs(p) + abs(pb)) * 1.02 + 1e-4)]
+        return [(pb, (sums + u * (abs(p) + abs(pb))) * 1.02 + 1e-4)]
     y = pb + res
-    e = u * (abs(p) + abs(pb) + abs(y))
+    e = sums + u * (abs(p) + abs(pb) + abs(y))
     if reader == "sum":
         return [(y, e * 1.02 + 1e-4)]
     if reader == "twice":
-        return [(y, e * 1.02 + 1e-4), (pb * pb, u * (2 * abs(pb) * (abs(p) + abs(pb)) + pb * pb) * 1.02 + 1e-4)]
+        return [(y, e * 1.02 + 1e-4), (pb * pb, (2 * abs(pb) * (sums + u * (abs(p) + abs(pb))) + u * pb * pb) * 1.02 + 1e-4)]
     std = np.sqrt(y.var(-1, keepdims=True) + 1e-12)
     h = (y - y.mean(-1, keepdims=True)) / std
     dh = (e + e.mean(-1, keepdims=True)) / std + abs(h) * np.sqrt((e * e).mean(-1, keepdims=True)) / std + u * abs(h)
@@ -78,12 +92,14 @@ def test_split(client, case):
     text = build(*spec)
     rng = np.random.default_rng(len(name))
     shapes = [tuple(int(d) for d in a.split("tensor<")[1].split(">")[0].split("x")[:-1]) for a in text[:text.index("->")].split("%arg")[1:]]
-    ins = [round_bf16(rng.standard_normal(s).astype(np.float32) / (np.float32(spec[1]) ** 0.25 if i < 2 else 1)) for i, s in enumerate(shapes)]
+    ins = [rng.standard_normal(s).astype(np.float32) / (np.float32(spec[1]) ** 0.25 if i < 2 else np.float32(1)) for i, s in enumerate(shapes)]
+    if not spec[5]:
+        ins = [round_bf16(a) for a in ins]
     want = exact_and_bound(spec, *ins)
     print("case", name, flush=True)
     exe = client.compile_and_load(text)
     for _ in range(2):
-        got = [runner.download(o) for o in exe.execute(runner.upload(client, ins, ["bf16"] * len(ins)))]
+        got = [runner.download(o) for o in exe.execute(runner.upload(client, ins, ["f32" if spec[5] else "bf16"] * len(ins)))]
         assert len(got) == len(want)
         for g, (w, bound) in zip(got, want):
             assert np.all(np.abs(np.asarray(g, np.float64) - w) <= bound), (name, float(np.max(np.abs(g - w) / bound)))
