@@ -76,6 +76,9 @@ typedef struct {
   // > 1 (mi355_gemm_split_parts): C holds that many float32 partial results one after the other, and whoever reads it adds
   // them in order and rounds the sum to out_dtype; no bias, no act
   int split;
+  // > 0 (small fp32 products only): the batches are groups of `heads`, and C is [group][m][head][n] instead of
+  // [group][head][m][n], i.e. the heads of a row lie side by side
+  int heads;
 } mi355_gemm_desc;
 int mi355_gemm_split_parts(const mi355_gemm_desc* d);
 int mi355_gemm_few_split(const mi355_gemm_desc* d);

@@ -196,6 +196,7 @@ struct SmallArgs {
   long long M, N;
   int batch1;
   int relu;            // the stored value is maximum(sum + bias, 0)
+  int heads;           // > 0: batch g * heads + h is stored as C[g][m][h][n] (no addend)
 };
 
 // The MFMA contraction does not care which k a lane's operand slot stands for as long as A and B agree, so a
@@ -318,7 +319,9 @@ __device__ __forceinline__ void smallGemmTileBody(const SmallArgs& g, unsigned b
     red[w][row * T + r] = acc[i];
   }
   __syncthreads();
-  float* C = g.c + (long long)bz * g.M * g.N;
+  // heads of a row side by side: the copy that gathered them behind the product (3.1 MB: 5.1 us, of a layer's 196) is gone
+  float* C = g.c + (g.heads ? (bz / g.heads * g.M * g.heads + bz % g.heads) * g.N : (long long)bz * g.M * g.N);
+  const long long ldc = g.heads ? g.heads * g.N : g.N;
   const float* D = g.addend ? g.addend + (long long)bz * g.M * g.N : nullptr;
   for (int e = threadIdx.x; e < T * T; e += 256) {
     const long long row = m0 + e / T, col = n0 + e % T;
@@ -326,7 +329,7 @@ __device__ __forceinline__ void smallGemmTileBody(const SmallArgs& g, unsigned b
       float sum = (red[0][e] + red[1][e]) + (red[2][e] + red[3][e]);
       if (D) sum += D[row * g.N + col];
       const float v = g.bias ? sum + g.bias[col] : sum;
-      C[row * g.N + col] = g.relu ? ((v > 0.f || v != v) ? v : 0.f) : v;   // maximum(v, 0): NaN stays NaN, -0 becomes +0
+      C[row * ldc + col] = g.relu ? ((v > 0.f || v != v) ? v : 0.f) : v;   // maximum(v, 0): NaN stays NaN, -0 becomes +0
     }
   }
 }
@@ -1293,6 +1296,7 @@ static bool fillSmall(SmallArgs& g, const void* addend, const mi355_gemm_desc* d
   g.M = d1->M; g.N = d1->N;
   g.batch1 = (int)d1->batch1;
   g.relu = d1->act == 2;
+  g.heads = d1->heads;
   return true;
 }
 
@@ -1343,6 +1347,7 @@ int mi355_gemm_small_sum(const mi355_gemm_desc* d1, const void* a1, const void* 
   g.M = d1->M; g.N = d1->N;
   g.batch1 = (int)d1->batch1;
   g.relu = d1->act == 2;
+  g.heads = d1->heads;
   dim3 grid((unsigned)((d1->N + t - 1) / t), (unsigned)((d1->M + t - 1) / t), (unsigned)(d1->batch0 * d1->batch1));
   if (t == 16) gemm_f32_small<16><<<grid, 256, 0, (hipStream_t)s>>>(g);
   else gemm_f32_small<32><<<grid, 256, 0, (hipStream_t)s>>>(g);
@@ -1381,6 +1386,7 @@ int mi355_gemm(const mi355_gemm_desc* d, const void* a, const void* b, void* c, 
   }
   if (d->act == 2 ? !smallGemmTile(d) : (d->act && d->out_dtype != 1)) return 2;   // epilogues: GELU for bf16 results, maximum(x, 0) for small fp32 products
   if (smallGemmTile(d)) return mi355_gemm_small_sum(d, a, b, nullptr, nullptr, nullptr, c, bias, nullptr, s);
+  if (d->heads) return 2;
   mi355_conv_desc cd;
   // strided views may start anywhere; the implicit-GEMM loaders issue 16-byte loads
   if (gemmAsPointwiseConv(d, &cd) && (((uintptr_t)a | (uintptr_t)b) & 15) == 0) {

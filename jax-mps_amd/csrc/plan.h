@@ -45,6 +45,7 @@ struct GemmDesc {   // C[b0,b1] = A[b0,b1] x B[b0,b1]; operands addressed throug
   int act = 0;                                     // 1: tanh-form GELU epilogue with the constants below; 2: maximum(x, 0)
   float actA = 0.f, actB = 0.f, actC = 0.f;
   int split = 1;                                   // > 1: stored as that many float32 partial results (mi355_gemm_desc::split)
+  int64_t heads = 0;                               // > 0: C is [group][m][head][n] (mi355_gemm_desc::heads)
 };
 
 struct ConvDesc {   // StableHLO convolution with arbitrary dimension numbers (<= 3 spatial dims, kernels specialise 2)

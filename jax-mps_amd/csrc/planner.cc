@@ -1943,8 +1943,22 @@ class Planner {
         if (y != produced && y->type == produced->type && hasStorage(y)) accumulate = u, addendV = y;
       }
     }
+    // [batch, head, row, feature] -> transpose to [batch, row, head, feature] -> reshape that something needs in memory (the
+    // attention heads merged for the next projection), nothing else reading any of them: stored in that order by a small fp32 product
+    Op *headsApart = nullptr, *headsMerged = nullptr;
+    if (!second && !biasAdd && !fuseAct && !relu && !accumulate && loopDepth_ == 0 && c->type.numel() > 0 && c->type.rank() == 4 && dp.rhsFreeDims == 1 &&
+        op->ints("lhs_batch").size() == 2 && c->users.size() == 1 && g.inType == DType::F32 && g.outType == DType::F32) {
+      mi355_gemm_desc small = toAbi(g);
+      Op* u = c->users[0];
+      if (mi355_gemm_is_small(&small) && u->name == "transpose" && u->parent == op->parent && u->ints("dims") == std::vector<int64_t>{0, 2, 1, 3} &&
+          u->result()->users.size() == 1 && !needMat_[u->result()]) {
+        Op* r = u->result()->users[0];
+        if (r->name == "reshape" && r->parent == op->parent && needMat_[r->result()] && !hasStorage(r->result())) headsApart = u, headsMerged = r;
+      }
+    }
     int sid = newStorage(c->type.bytes());
-    bind(produced, sid);
+    bind(headsMerged ? headsMerged->result() : produced, sid);   // (only its last form is ever read)
+    if (headsMerged) emitted_.insert(headsApart), emitted_.insert(headsMerged);
     if (sumAdd) emitted_.insert(sumAdd);
     if (c->type.numel() == 0) return;
     int t = ++time_;
@@ -1952,13 +1966,14 @@ class Planner {
     s.kind = Step::Gemm;
     s.time = t;
     s.label = "dot_general " + a->type.str() + " x " + b->type.str() + (second ? " + " + second->operands[0]->type.str() + " x " + second->operands[1]->type.str() : "") +
-              (biasV ? " + bias" : "") + (fuseAct ? " + gelu" : "") + (relu ? " + relu" : "") + (accumulate ? " + tensor" : "");
+              (biasV ? " + bias" : "") + (fuseAct ? " + gelu" : "") + (relu ? " + relu" : "") + (accumulate ? " + tensor" : "") + (headsMerged ? ", heads merged" : "");
     if (accumulate) {
       s.addend = ref(storageOf(addendV), t);
       storage_[accumulate->result()] = sid;   // the step writes the sum; nothing reads the bare product, so the buffer still holds one value
       emitted_.insert(accumulate);
     }
     s.gemm = g;
+    if (headsMerged) s.gemm.heads = c->type.dims[1];
     if (relu) {
       s.gemm.act = 2;
       bind(relu->result(), sid);   // the step writes the activation; nothing reads the value before it
@@ -3025,6 +3040,7 @@ mi355_gemm_desc toAbi(const GemmDesc& g) {
   d.out_dtype = abiDtypeCode(g.outType);
   d.act = g.act; d.act_a = g.actA; d.act_b = g.actB; d.act_c = g.actC;
   d.split = g.split;
+  d.heads = (int)g.heads;
   return d;
 }
 

@@ -1,0 +1,67 @@
+"""A small float32 attention product whose heads are merged for the next projection is stored with a row's heads side by side:
+tile edges of both tile sizes, one batch, either layout of the values, the merged rows read by a product, returned,
+or both; and what keeps the order of its batches (one head, a product that is not small, another permutation, a second reader of
+the product)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+# name, batch, heads, rows, keys, features, values as [batch, key, head, feature], reader, stored with heads side by side
+CASES = [
+    ("odd", 2, 3, 17, 33, 18, True, "product", True),
+    ("values-per-head", 2, 3, 16, 32, 16, False, "product", True),
+    ("one-batch", 1, 4, 37, 37, 64, True, "product", True),
+    ("one-head", 3, 1, 5, 7, 9, True, "product", False),
+    ("wide-tiles", 8, 12, 128, 128, 64, True, "product", True),
+    ("returned", 2, 5, 31, 8, 12, True, "returned", True),
+    ("returned-and-read", 2, 5, 31, 8, 12, True, "both", True),
+    ("not-small", 8, 8, 256, 512, 64, True, "product", False),
+    ("rows-last", 2, 3, 16, 24, 16, True, "rows-last", False),
+    ("product-returned", 2, 3, 17, 33, 18, True, "product-returned", False),
+]
+
+
+def build(batch, heads, rows, keys, features, by_key, reader, merged):
+    from jax_mps_amd.shlo.builder import Builder
+    b = Builder("gemm_heads")
+    p = b.arg((batch, heads, rows, keys), "f32")
+    v = b.arg((batch, keys, heads, features) if by_key else (batch, heads, keys, features), "f32")
+    w = b.arg((heads * features, 24), "f32")
+    y = b.dot_general(p, v, ([3], [1 if by_key else 2]), ([0, 1], [0, 2 if by_key else 1]))
+    if reader == "rows-last":
+        t = b.reshape(b.transpose(y, [0, 3, 1, 2]), (batch, features * heads, rows))
+        b.ret(b.dot_general(t, w, ([1], [0])))
+        return b.text()
+    t = b.reshape(b.transpose(y, [0, 2, 1, 3]), (batch, rows, heads * features))
+    z = b.dot_general(t, w, ([2], [0]))
+    b.ret(*{"product": [z], "returned": [t], "both": [t, z], "product-returned": [y, z]}[reader])
+    return b.text()
+
+
+def exact(case, p, v, w):
+    name, batch, heads, rows, keys, features, by_key, reader, merged = case
+    p, v, w = (a.astype(np.float64) for a in (p, v, w))
+    y = p @ (v.transpose(0, 2, 1, 3) if by_key else v)
+    if reader == "rows-last":
+        return [np.einsum("bkr,kn->brn", y.transpose(0, 3, 1, 2).reshape(batch, features * heads, rows), w)]
+    t = y.transpose(0, 2, 1, 3).reshape(batch, rows, heads * features)
+    return {"product": [t @ w], "returned": [t], "both": [t, t @ w], "product-returned": [y, t @ w]}[reader]
+
+
+@pytest.mark.parametrize("case", CASES, ids=[c[0] for c in CASES])
+def test_heads(client, case):
+    from jax_mps_amd import runner
+    name, batch, heads, rows, keys, features, by_key, reader, merged = case
+    rng = np.random.default_rng(rows)
+    shapes = [(batch, heads, rows, keys), (batch, keys, heads, features) if by_key else (batch, heads, keys, features), (heads * features, 24)]
+    ins = [rng.standard_normal(s).astype(np.float32) for s in shapes]
+    print("case", name, flush=True)
+    exe = client.compile_and_load(build(*case[1:]))
+    for _ in range(2):
+        got = [runner.download(o) for o in exe.execute(runner.upload(client, ins, ["f32"] * 3))]
+        for g, want, magnitude in zip(got, exact(case, *ins), exact(case, *map(np.abs, ins))):
+            # a float32 sum of n products is within n * 2^-24 of their absolute sum, in any order; here of keys, then of heads * features
+            bound = (keys + heads * features) * 2.0 ** -24 * magnitude
+            assert g.shape == want.shape
+            assert np.all(np.abs(g - want) <= bound), (name, float(np.max(np.abs(g - want) / bound)))
