@@ -962,10 +962,7 @@ ConvChoice choose(const mi355_conv_desc* d, long long tapsVisited = -1, int shar
   static const int minSplitTiles = getenv("MI355X_CONV_MIN_SPLIT_KTILES") ? atoi(getenv("MI355X_CONV_MIN_SPLIT_KTILES")) : 1;
   // (measured: splitting pays even for a short K, the shorter dependent chain per workgroup outweighs the fold launch)
   static const int splitFactor = getenv("MI355X_CONV_SPLIT_FACTOR") ? atoi(getenv("MI355X_CONV_SPLIT_FACTOR")) : 3;
-  // k-tiles a split keeps at least: with 12 (6 where there are few tiles) instead of 8 (4) the partial sums are fewer; ResNet
-  // train steps of batch 8 to 40 take 3 to 15 % less, forward passes up to 4 %, batch 48 and more the same.
-  constexpr int kSplitTiles = 12, kSplitTilesFew = 6;
-  if (tiles * (c.amode == 2 ? 2 : splitFactor) <= target && c.kTiles >= minSplitTiles) split = (int)std::min<long long>(target / tiles, std::max(1, c.kTiles / (tiles < 64 ? kSplitTilesFew : kSplitTiles)));
+  if (tiles * (c.amode == 2 ? 2 : splitFactor) <= target && c.kTiles >= minSplitTiles) split = (int)std::min<long long>(target / tiles, std::max(1, c.kTiles / (tiles < 64 ? 4 : 8)));
   split = std::max(1, std::min(split, 256));
   static const bool xcdSplit = getenv("MI355X_CONV_XCD_SPLIT") && getenv("MI355X_CONV_XCD_SPLIT")[0] == '1';
   if (xcdSplit && split >= 16) split = split / 8 * 8;   // whole groups of K ranges per XCD, so that no XCD runs a workgroup more than the others
