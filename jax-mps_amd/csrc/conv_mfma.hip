@@ -779,26 +779,19 @@ __global__ void __launch_bounds__(256) conv_fold_few(const float* __restrict__ p
 }
 
 // The fold of a split convolution whose output's column sums and sums of squares are wanted (batch-norm statistics): a
-// workgroup folds 16 * rowSteps rows of 64 columns, four columns a lane, and adds up its rows on the way, so that no pass
+// workgroup folds 16 rows of 64 columns, four columns a lane, and adds up its rows on the way, so that no pass
 // of its own reads the output again (batch 16, 32 x 32 x 64: fold 5.7 and pass 4.7 us apart, 6.5 together; the forward pass
 // of ResNet18 546 -> 505 us).  The partials of an element are added in the order of conv_fold_few
 // (at most eight) or conv_fold_partials (more), so the output has the same bits with and without statistics.
 constexpr int kFoldRows = 16, kFoldCols = 64;
-// rows of statistics partials, and rows per lane: more rows a workgroup while 512 workgroups are left
-__host__ __device__ inline int foldRowSteps(long long M, long long N) {
-  const long long groups = (M + kFoldRows - 1) / kFoldRows * ((N + kFoldCols - 1) / kFoldCols);
-  return groups >= 4096 ? 8 : groups >= 2048 ? 4 : groups >= 1024 ? 2 : 1;
-}
 
 template <bool MANY>
-__global__ void __launch_bounds__(256) conv_fold_stats(const float* __restrict__ part, float* __restrict__ out, ConvP p, int rowSteps, int statRows) {
+__global__ void __launch_bounds__(256) conv_fold_stats(const float* __restrict__ part, float* __restrict__ out, ConvP p, int statRows) {
   __shared__ float sums[2][kFoldRows][kFoldCols + 4];
   const int quad = threadIdx.x & 15, r = threadIdx.x >> 4, n = (int)blockIdx.y * kFoldCols + quad * 4;   // p.N % 4 == 0 (checked by the launcher)
   const long long total = (long long)p.M * p.N;
   float4 sum = make_float4(0.f, 0.f, 0.f, 0.f), sq = sum;
-  for (int k = 0; k < rowSteps; ++k) {
-    const int m = ((int)blockIdx.x * rowSteps + k) * kFoldRows + r;
-    if (m >= p.M || n >= p.N) break;
+  if (const int m = (int)blockIdx.x * kFoldRows + r; m < p.M && n < p.N) {
     const long long i = (long long)m * p.N + n;
     const float* at = part + i;
     float4 s;
@@ -1189,10 +1182,10 @@ static int launchPart(const ConvPart& part, const void* lhs, const void* rhs, vo
       if (bias || part.outOffset || p.N % 4 != 0 || (((uintptr_t)workspace | (uintptr_t)dst) & 15) != 0) return 5;   // (mi355_conv_stats_rows promised otherwise)
       p.statSum = statSum;
       p.statSq = statSq;
-      const int steps = foldRowSteps(p.M, p.N), rows = (p.M + kFoldRows * steps - 1) / (kFoldRows * steps);
+      const int rows = (p.M + kFoldRows - 1) / kFoldRows;
       const dim3 blocks((unsigned)rows, (unsigned)((p.N + kFoldCols - 1) / kFoldCols));
-      if (c.splitK > 8) conv_fold_stats<true><<<blocks, 256, 0, st>>>((const float*)workspace, dst, p, steps, rows);
-      else conv_fold_stats<false><<<blocks, 256, 0, st>>>((const float*)workspace, dst, p, steps, rows);
+      if (c.splitK > 8) conv_fold_stats<true><<<blocks, 256, 0, st>>>((const float*)workspace, dst, p, rows);
+      else conv_fold_stats<false><<<blocks, 256, 0, st>>>((const float*)workspace, dst, p, rows);
     } else if (c.splitK <= 8 && p.N % 4 == 0 && ((uintptr_t)workspace & 15) == 0)
       conv_fold_few<<<(unsigned)((total / 4 + 255) / 256), 256, 0, st>>>((const float*)workspace, dst, p);
     else
@@ -1222,10 +1215,7 @@ int mi355_conv_stats_rows(const mi355_conv_desc* d) {
   long long expect = d->O;
   for (int k = d->nsp - 1; k >= 0; --k) { if (d->outS[k] != expect) return 0; expect *= d->out[k]; }
   if (d->outB != expect) return 0;
-  if (c.splitK > 1) {
-    const int rows = kFoldRows * foldRowSteps(M, d->O);
-    return (int)((M + rows - 1) / rows);
-  }
+  if (c.splitK > 1) return (int)((M + kFoldRows - 1) / kFoldRows);
   return (int)((M + c.bm - 1) / c.bm);
 }
 

@@ -24,13 +24,13 @@ CASES = [
     ("short-k", 16, 352, 64, False, "norm", False),
     ("no-residual", 16, 768, 64, False, "bias", False),
     ("two-readers", 16, 768, 64, False, "twice", False),
-    ("f32-two-parts", 1000, 400, 516, False, "norm", True),
-    ("f32-eight-parts", 600, 1600, 644, False, "norm", True),
+    ("f32-two-parts", 1000, 272, 644, False, "norm", True),
+    ("f32-eight-parts", 600, 1076, 644, False, "norm", True),
     ("f32-ragged-k", 520, 804, 520, False, "rank-3", True),
     ("f32-k-contiguous", 1024, 768, 768, True, "norm", True),
     ("f32-stored", 1027, 768, 768, False, "sum", True),
-    ("f32-nine-parts", 600, 1744, 644, False, "norm", True),
-    ("f32-columns", 600, 1600, 646, False, "norm", True),
+    ("f32-nine-parts", 600, 1168, 644, False, "norm", True),
+    ("f32-columns", 600, 1076, 646, False, "norm", True),
     ("f32-no-residual", 1000, 400, 516, False, "bias", True),
     ("f32-two-readers", 1000, 400, 516, False, "twice", True),
 ]
